@@ -1,5 +1,6 @@
 // qv_truth.hip -- brute-force exact nearest neighbours (ground truth) on the GPU.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -252,13 +253,664 @@ __global__ void gt_query_check(const float* __restrict__ q, int64_t count, int32
   }
 }
 
+// ---- ground truth on the matrix cores ---------------------------------------
+//
+// A scan over base rows that only has to find, per query, the rows that may
+// still be among its k nearest: the products q.x of 32 rows and 32 queries at
+// a time come from MFMA, one compare against the query's threshold drops all
+// but a few hundred rows per query, and those few are ranked exactly
+// (gt_pick_kernel), so ids, distances and ties equal the direct kernels'.
+//   * 8-bit data: bytes shifted to int8 (a distance does not change), q.x exact
+//     in int32 (v_mfma_i32_32x32x32_i8).
+//   * float: rows and queries split into two bf16 parts (x = hi + lo + r,
+//     |r| <= 2^-17 |x|), q.x = hi hi + hi lo + lo hi in fp32
+//     (v_mfma_f32_32x32x16_bf16): only a bound.  Its error against the real
+//     q.x, the norms' and the ranked distance's own rounding together are
+//     below kGtEps (|q|^2 + |x|^2) for dim <= 128 (2^-15 |q||x| of dropped
+//     parts and 2^-15.4 of 3 x 128 accumulations, twice, plus 2^-16 for the
+//     sums of squares: under 2^-12.9), so a row is only dropped when its
+//     distance is above the threshold whatever the rounding.  The candidates'
+//     distances are the fp32 chain of the direct kernel.
+// Thresholds come from the rows already scanned.  Level 0 takes every S-th row
+// (S = 4^m, a few hundred rows) and keeps them all; level j the rows whose
+// number modulo S lies in [w, 4 w), w = 4^(j - 1), so every level scans three
+// times the rows of all before it, spread over the whole base, and about 3 k
+// of them pass the k-th distance found so far.  A list that overflows all the
+// same (data ordered against the period) sends the call to the direct kernels.
+//
+// What bounds it: the matrix pipes need 4 x 32 cycles per 32 x 32 pairs of 128
+// bytes (1.25 M of the last level's 3.1 M cycles at the sizes below), the rest
+// is the compare (8 max3 and a compare per 1,024 pairs), the candidates' path
+// and the barrier that ties a workgroup's waves to the slowest of them.  So
+// one tile of rows in LDS serves four query tiles per wave (two for float, 24
+// MFMA per operand pair) while the next is in flight in registers, and a
+// candidate costs no wait: it goes to a pool in LDS, 64 of them to the lists
+// in one round trip of counter atomics.  Two query tiles per wave and twice
+// the waves: 1.69 ms for the last level instead of 1.44 (float, one instead of
+// two: 0.74 instead of 0.48).
+// Measured, whole call: 10,000 queries x 1M x 128 uint8, k = 10: 2.4 ms
+// (18.8 ms with one query per lane and dot4); 2,001 x 500,001 x 96 float: 0.96
+// ms (12.1 ms with 8 queries per workgroup and fp32 FMA).
+
+typedef int32_t gt_i4 __attribute__((ext_vector_type(4)));
+typedef int32_t gt_i16 __attribute__((ext_vector_type(16)));
+typedef float gt_f16 __attribute__((ext_vector_type(16)));
+typedef __bf16 gt_b8 __attribute__((ext_vector_type(8)));
+
+constexpr int kGtRows = 64;          // base rows per LDS tile
+constexpr int64_t kGtBatch = 32768;  // queries per scan: the lists' memory (4 KB a query up to k = 16, 16 KB beyond)
+constexpr int kGtPool = 128;         // candidates a wave gathers in LDS before it appends them to the lists
+constexpr float kGtEps = 1.0f / 4096.0f;
+constexpr float kGtHuge = 1e37f;     // |x|^2 above this: the row or query is never dropped
+constexpr int kGtDrop = -(1 << 29);  // (8-bit) accumulator start of rows past the end
+
+struct ScanArgs {
+  const uint8_t* base;
+  int64_t row_bytes;
+  int64_t rows;         // rows of this level (gt_base_row)
+  int64_t period;       // S
+  int32_t shift;        // log2 w, -1 at level 0
+  int64_t nq;
+  int groups, slices;   // query groups, row slices (a multiple of 8)
+  const uint8_t* qp;    // packed queries, [padded nq][planes * KS * 32] bytes
+  const uint32_t* qn;   // |q|^2 (int32 or float bits), [padded nq]
+  const uint32_t* thr;  // accumulator threshold (int32 or float bits), [padded nq]
+  const uint64_t* tkey; // (8-bit) key no candidate may exceed, [padded nq]
+  uint32_t* cnt;        // [padded nq] candidates listed
+  uint64_t* list;       // [nq][cap] keys (8-bit) or row ids (float)
+  int cap;
+  int32_t* over;        // set when a list overflows: the call is lost, its scans end early
+};
+
+// Base row of a level's row i: every S-th row at level 0, else row i of the
+// runs [S b + w, S b + 4 w).
+__device__ __forceinline__ int64_t gt_base_row(const ScanArgs& a, uint32_t i) {
+  if (a.shift < 0) return (int64_t)i * a.period;
+  const uint32_t u = i >> a.shift, b = u / 3u;
+  return (int64_t)b * a.period + ((int64_t)(u - 3u * b + 1u) << a.shift) + (int64_t)(i & ((1u << a.shift) - 1u));
+}
+
+template <class T>
+struct GtKind {
+  static constexpr bool kFloat = sizeof(T) == 4;
+  static constexpr int kPlanes = kFloat ? 2 : 1;
+  static constexpr int kPieceBytes = kFloat ? 32 : 16;  // source bytes behind one 16-byte LDS piece
+  using Acc = std::conditional_t<kFloat, gt_f16, gt_i16>;
+  using One = std::conditional_t<kFloat, float, int32_t>;
+};
+
+// LDS bytes of one tile row: its planes, then 16 bytes so that the row is an
+// odd number of 16-byte pieces (lanes reading one piece of 32 rows spread over
+// all banks).
+template <class T>
+constexpr int gt_row_lds(int KS) {
+  return GtKind<T>::kPlanes * KS * 32 + 16;
+}
+template <class T>
+constexpr int gt_scan_lds(int KS, int QT) {
+  return 2 * kGtRows * (gt_row_lds<T>(KS) + 8) + 4 * kGtPool * 12 + (GtKind<T>::kFloat ? 0 : 128 * QT * 12) + 8;
+}
+
+// bf16 parts of 8 floats: hi rounded to nearest, lo the rounded rest.
+__device__ __forceinline__ void gt_split(const float (&x)[8], gt_b8& hi, gt_b8& lo) {
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const __bf16 h = (__bf16)x[j];
+    hi[j] = h;
+    lo[j] = (__bf16)(x[j] - (float)h);
+  }
+}
+
+// Four source words of a row of nwords 32-bit words from w0 on, zero past its
+// end.
+__device__ __forceinline__ gt_i4 gt_words(const uint32_t* row, int w0, int nwords) {
+  typedef gt_i4 gt_i4u __attribute__((aligned(4)));  // rows are 4-byte aligned
+  gt_i4 v = {0, 0, 0, 0};
+  if (w0 + 4 <= nwords) {
+    v = *reinterpret_cast<const gt_i4u*>(row + w0);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (w0 + e < nwords) v[e] = (int32_t)row[w0 + e];
+  }
+  return v;
+}
+
+// uint8 words as int8 (x - 128), zero past the row's end.
+template <class T>
+__device__ __forceinline__ gt_i4 gt_shift(gt_i4 v, int w0, int nwords) {
+  if constexpr (!std::is_signed<T>::value && sizeof(T) == 1) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = w0 + e < nwords ? (int32_t)((uint32_t)v[e] ^ 0x80808080u) : 0;
+  }
+  return v;
+}
+
+// Queries into the scan's operand layout, with their norms, an open threshold
+// and an empty list; *lost is set when an 8-bit index's query is not a whole
+// number of the element type's range (the direct kernel takes those).  One
+// wave per query slot; slots past nq never match.
+template <class T, int KS>
+__global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ queries, int64_t nq, int dim,
+                                                     uint8_t* __restrict__ qp, uint32_t* __restrict__ qn,
+                                                     uint32_t* __restrict__ thr, uint64_t* __restrict__ tkey,
+                                                     uint32_t* __restrict__ cnt, int32_t* __restrict__ lost) {
+  using K = GtKind<T>;
+  const int lane = lane_id();
+  const int64_t q = blockIdx.x;
+  const bool live = q < nq;
+  uint8_t* const out = qp + q * (int64_t)(K::kPlanes * KS * 32);
+  if constexpr (K::kFloat) {
+    float s = 0.f;
+    if (lane < KS * 2) {
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int i = lane * 8 + j;
+        x[j] = live && i < dim ? queries[q * dim + i] : 0.f;
+        s = __fmaf_rn(x[j], x[j], s);
+      }
+      gt_b8 hi, lo;
+      gt_split(x, hi, lo);
+      *reinterpret_cast<gt_b8*>(out + lane * 16) = hi;
+      *reinterpret_cast<gt_b8*>(out + KS * 32 + lane * 16) = lo;
+    }
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (lane == 0) {
+      qn[q] = __float_as_uint(s);
+      thr[q] = __float_as_uint(live ? -__int_as_float(0x7f800000) : __int_as_float(0x7f800000));
+    }
+  } else {
+    const float lo = std::is_signed<T>::value ? -128.f : 0.f, hi = std::is_signed<T>::value ? 127.f : 255.f;
+    constexpr int kShift = std::is_signed<T>::value ? 0 : 128;
+    int32_t s = 0;
+    bool wrong = false;
+    for (int w = lane; w < KS * 8; w += kWave) {
+      uint32_t packed = 0;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int i = 4 * w + e;
+        if (live && i < dim) {
+          const float v = queries[q * dim + i];
+          if (!(v >= lo && v <= hi && v == rintf(v))) wrong = true;
+          packed |= ((uint32_t)((int)v - kShift) & 0xffu) << (8 * e);
+        }
+      }
+      s = __builtin_amdgcn_sdot4((int)packed, (int)packed, s, false);
+      reinterpret_cast<uint32_t*>(out)[w] = packed;
+    }
+    if (wrong) *lost = 1;
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (lane == 0) {
+      qn[q] = (uint32_t)s;
+      thr[q] = (uint32_t)(live ? INT32_MIN : INT32_MAX);
+    }
+  }
+  if (lane == 0) {
+    tkey[q] = kPadKey;
+    cnt[q] = 0;
+  }
+}
+
+// One workgroup: 4 waves of QT x 32 queries each, over the row tiles of one
+// slice.  Rows are D's rows and queries its columns, so a lane's 16 sums all
+// belong to one query and one register holds its threshold; the accumulators
+// start at minus half the rows' norms, so that "sum >= threshold" is the whole
+// test.  Workgroups that share a slice run on one XCD (round-robin over 8 by
+// workgroup number), whose L2 then serves its rows to all query groups.
+template <class T, int KS, int QT>
+__global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
+  using K = GtKind<T>;
+  using Acc = typename K::Acc;
+  using One = typename K::One;
+  constexpr int P = K::kPlanes;
+  constexpr int kPieces = KS * 2;                                                // per plane and row
+  constexpr int kGroup = kPieces <= 4 ? 4 : (kPieces <= 8 ? 8 : 16);             // lanes per staged row
+  constexpr int kRounds = kGtRows * kGroup / 256;
+  constexpr int kLoads = K::kPieceBytes / 16;
+  constexpr int kStride = gt_row_lds<T>(KS);
+  extern __shared__ __align__(16) char smem[];
+  char* const tile = smem;                                                       // [2][kGtRows][kStride]
+  One* const start = reinterpret_cast<One*>(smem + 2 * kGtRows * kStride);       // [2][kGtRows]
+  One* const odds = start + 2 * kGtRows;                                         // (8-bit) |x|^2 & 1
+  // one wave's pool: level rows, query slots of the wave and (8-bit) sums
+  int32_t* const pools = reinterpret_cast<int32_t*>(odds + 2 * kGtRows);         // [4 waves][3][kGtPool]
+  uint32_t* const pool_at = reinterpret_cast<uint32_t*>(pools + (threadIdx.x / kWave) * 3 * kGtPool);
+  int32_t* const pool_q = reinterpret_cast<int32_t*>(pool_at + kGtPool);
+  int32_t* const pool_sum = pool_q + kGtPool;
+  // (8-bit) the workgroup's queries' key limits and norms
+  uint64_t* const tkey = reinterpret_cast<uint64_t*>(pools + 4 * 3 * kGtPool);
+  int32_t* const qnorm = reinterpret_cast<int32_t*>(tkey + 128 * QT);
+  int32_t* const ended = reinterpret_cast<int32_t*>(smem + gt_scan_lds<T>(KS, QT) - 8);  // [2]
+
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  const int col = lane & 31, half = lane >> 5;
+  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int group = j % a.groups, slice = (j / a.groups) * 8 + xcd;
+  const int64_t q0 = ((int64_t)group * 4 + wave) * (32 * QT) + col;
+  const int64_t tiles = (a.rows + kGtRows - 1) / kGtRows;
+  const int nwords = (int)(a.row_bytes / 4);
+
+  gt_i4 b[QT][P][KS];
+  One thr[QT];
+#pragma unroll
+  for (int t = 0; t < QT; t++) {
+    const uint8_t* const src = a.qp + (q0 + 32 * t) * (int64_t)(P * KS * 32) + half * 16;
+#pragma unroll
+    for (int p = 0; p < P; p++)
+#pragma unroll
+      for (int s = 0; s < KS; s++) b[t][p][s] = *reinterpret_cast<const gt_i4*>(src + (p * KS + s) * 32);
+    const uint32_t bits = a.thr[q0 + 32 * t];
+    if constexpr (K::kFloat) thr[t] = __uint_as_float(bits);
+    else thr[t] = (int32_t)bits;
+  }
+
+  const int piece = tid % kGroup;
+  gt_i4 in[kRounds][kLoads];
+  auto request = [&](int64_t t) {
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) {
+      const int64_t i = t * kGtRows + tid / kGroup + r * (256 / kGroup);
+      const bool ok = piece < kPieces && i < a.rows;
+      const uint32_t* const src = reinterpret_cast<const uint32_t*>(a.base + gt_base_row(a, ok ? (uint32_t)i : 0u) * a.row_bytes);
+#pragma unroll
+      for (int l = 0; l < kLoads; l++)
+        in[r][l] = ok ? gt_words(src, piece * (K::kPieceBytes / 4) + 4 * l, nwords) : gt_i4{0, 0, 0, 0};
+    }
+  };
+  auto stage = [&](int64_t t, int buf) {
+#pragma unroll
+    for (int r = 0; r < kRounds; r++) {
+      const int row = tid / kGroup + r * (256 / kGroup);
+      char* const dst = tile + (buf * kGtRows + row) * kStride + piece * 16;
+      const bool live = t * kGtRows + row < a.rows;
+      One s = 0;
+      if constexpr (K::kFloat) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          x[e] = __int_as_float(in[r][e / 4][e % 4]);
+          s = __fmaf_rn(x[e], x[e], s);
+        }
+        for (int off = 1; off < kGroup; off <<= 1) s += __shfl_xor(s, off);
+        const bool keep = !(s <= kGtHuge);  // never dropped: zero row, accumulators at +inf
+        if (keep) {
+#pragma unroll
+          for (int e = 0; e < 8; e++) x[e] = 0.f;
+        }
+        gt_b8 hi, lo;
+        gt_split(x, hi, lo);
+        if (piece < kPieces) {
+          *reinterpret_cast<gt_b8*>(dst) = hi;
+          *reinterpret_cast<gt_b8*>(dst + KS * 32) = lo;
+        }
+        if (piece == 0) {
+          const float inf = __int_as_float(0x7f800000);
+          start[buf * kGtRows + row] = !live ? -inf : (keep ? inf : -0.5f * (1.f - kGtEps) * s);
+        }
+      } else {
+        const gt_i4 v = gt_shift<T>(in[r][0], piece * 4, live ? nwords : 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s = __builtin_amdgcn_sdot4(v[e], v[e], s, false);
+        for (int off = 1; off < kGroup; off <<= 1) s += __shfl_xor(s, off);
+        if (piece < kPieces) *reinterpret_cast<gt_i4*>(dst) = v;
+        if (piece == 0) {
+          odds[buf * kGtRows + row] = s & 1;
+          start[buf * kGtRows + row] = live ? -((s + 1) >> 1) : kGtDrop;
+        }
+      }
+    }
+  };
+
+  // This wave's pooled candidates into their queries' lists, 64 at a time: one
+  // round trip of counter atomics for 64 of them.
+  int pooled = 0;
+  auto flush = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    // a lost call adds nothing more (its counters would only be fought over)
+    if (pooled > 0 && __hip_atomic_load(a.over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) pooled = 0;
+    for (int i = lane; i < pooled; i += kWave) {
+      const uint32_t at = pool_at[i];
+      const int lq = wave * 32 * QT + pool_q[i];
+      const int64_t q = (int64_t)group * (128 * QT) + lq;
+      uint64_t entry = 0;
+      bool take = q < a.nq && (int64_t)at < a.rows;
+      if (take) entry = (uint64_t)gt_base_row(a, at);
+      if constexpr (!K::kFloat) {
+        const int32_t dist = qnorm[lq] - pool_sum[i];
+        entry |= (uint64_t)__float_as_uint((float)dist) << 32;
+        take = take && entry <= tkey[lq];
+      }
+      if (take) {
+        const uint32_t pos = atomicAdd(a.cnt + q, 1u);
+        if (pos < (uint32_t)a.cap) a.list[q * a.cap + pos] = entry;
+        else *a.over = 1;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    pooled = 0;
+  };
+
+  // The rows of one 32 x 32 tile that reach their query's threshold, into the
+  // pool, without a wait: 8-bit candidates leave with |q|^2 - dist = 2 sum +
+  // (|x|^2 & 1) (odd: the rows' norm parities), which flush turns into the key.
+  auto harvest = [&](const Acc& d, One limit, int qt, int rt, uint32_t odd, int64_t t) {
+    const uint32_t at = (uint32_t)(t * kGtRows) + (uint32_t)(rt * 32 + 4 * half);  // level row of element 0 (< 2^31)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const bool take = !(d[i] < limit);
+      const uint64_t m = __ballot(take);
+      if (m != 0) {
+        const int row = 8 * (i / 4) + (i & 3);
+        if (take) {
+          const int to = pooled + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+          pool_at[to] = at + row;
+          pool_q[to] = 32 * qt + col;
+          if constexpr (!K::kFloat) pool_sum[to] = 2 * d[i] + (int32_t)((odd >> row) & 1u);
+        }
+        pooled += (int)__popcll(m);
+        if (pooled > kGtPool - kWave) flush();
+      }
+    }
+  };
+
+  int64_t t = slice;
+  if (t >= tiles) return;  // the whole workgroup
+  request(t);
+  if constexpr (!K::kFloat) {
+    for (int i = tid; i < 128 * QT; i += 256) {
+      tkey[i] = a.tkey[(int64_t)group * (128 * QT) + i];
+      qnorm[i] = (int32_t)a.qn[(int64_t)group * (128 * QT) + i];
+    }
+  }
+  stage(t, 0);
+  __syncthreads();
+  int buf = 0;
+  while (true) {
+    const int64_t tn = t + a.slices;
+    const int32_t lost = __hip_atomic_load(a.over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tn < tiles) request(tn);
+    uint64_t parity = 0;
+    if constexpr (!K::kFloat) parity = __ballot(odds[buf * kGtRows + lane] != 0);
+#pragma unroll 1
+    for (int rt = 0; rt < kGtRows / 32; rt++) {
+      const char* const arow = tile + (buf * kGtRows + rt * 32 + col) * kStride + half * 16;
+      const int r0 = buf * kGtRows + rt * 32;
+      gt_i4 av[P][KS];
+#pragma unroll
+      for (int p = 0; p < P; p++)
+#pragma unroll
+        for (int s = 0; s < KS; s++) av[p][s] = *reinterpret_cast<const gt_i4*>(arow + (p * KS + s) * 32);
+      // D element 4 g + e of a lane: row 8 g + 4 half + e of the tile
+      Acc c;
+#pragma unroll
+      for (int g = 0; g < 4; g++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) c[4 * g + e] = start[r0 + 8 * g + 4 * half + e];
+      Acc d[QT];
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++) {
+          const Acc& in_c = s == 0 ? c : d[qt];
+          if constexpr (K::kFloat) {
+            const gt_b8 ah = __builtin_bit_cast(gt_b8, av[0][s]), al = __builtin_bit_cast(gt_b8, av[P - 1][s]);
+            const gt_b8 bh = __builtin_bit_cast(gt_b8, b[qt][0][s]), bl = __builtin_bit_cast(gt_b8, b[qt][P - 1][s]);
+            d[qt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, in_c, 0, 0, 0);
+            d[qt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, d[qt], 0, 0, 0);
+            d[qt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, d[qt], 0, 0, 0);
+          } else {
+            d[qt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[0][s], b[qt][0][s], in_c, 0, 0, 0);
+          }
+        }
+      }
+      bool pass[QT], any = false;
+#pragma unroll
+      for (int qt = 0; qt < QT; qt++) {
+        One top = d[qt][0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) {
+          if constexpr (K::kFloat) top = fmaxf(top, d[qt][i]);
+          else top = max(top, d[qt][i]);
+        }
+        pass[qt] = !(top < thr[qt]);
+        any |= pass[qt];
+      }
+      if (__ballot(any) == 0) continue;
+      uint32_t hits = 0;
+#pragma unroll
+      for (int qt = 0; qt < QT; qt++) hits |= __ballot(pass[qt]) != 0 ? 1u << qt : 0u;
+      uint32_t odd = 0;
+      if constexpr (!K::kFloat) odd = (uint32_t)(parity >> (rt * 32)) >> (4 * half);
+      // one copy of the harvest for every query tile (its code, not its moves, is the cost)
+#pragma unroll 1
+      while (hits != 0) {
+        const int qt = __builtin_ctz(hits);
+        hits &= hits - 1;
+        Acc x = d[0];
+        One limit = thr[0];
+#pragma unroll
+        for (int o = 1; o < QT; o++) {
+          if (qt == o) {
+            x = d[o];
+            limit = thr[o];
+          }
+        }
+        harvest(x, limit, qt, rt, odd, t);
+      }
+    }
+    if (tn >= tiles) break;
+    stage(tn, buf ^ 1);
+    if (tid == 0) ended[buf ^ 1] = lost;
+    __syncthreads();
+    buf ^= 1;
+    t = tn;
+    if (ended[buf]) break;  // the same word for every wave
+  }
+  flush();
+}
+
+// The k nearest of each query's listed rows, one wave per query: float rows
+// get their distance here (the direct kernel's fp32 chain over the
+// dimensions).  Before the last level: the threshold for the next one, and a
+// list of just these; at the last: the results.
+template <class T>
+__global__ __launch_bounds__(256) void gt_pick_kernel(const uint8_t* __restrict__ base, int64_t row_bytes, int dim,
+                                                      const float* __restrict__ queries, int64_t nq, int k,
+                                                      const uint32_t* __restrict__ qn, uint32_t* __restrict__ thr,
+                                                      uint64_t* __restrict__ tkey, uint32_t* __restrict__ cnt,
+                                                      uint64_t* __restrict__ list, int cap, bool last,
+                                                      int32_t* __restrict__ ids, float* __restrict__ dists) {
+  __shared__ float qs[4][128];
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int64_t q = (int64_t)blockIdx.x * 4 + wave;
+  constexpr bool kFloat = sizeof(T) == 4;
+  if constexpr (kFloat) {
+    for (int i = lane; i < dim; i += kWave) qs[wave][i] = q < nq ? queries[q * dim + i] : 0.f;
+    __syncthreads();
+  }
+  if (q >= nq) return;
+  const int m = (int)min(cnt[q], (uint32_t)cap);
+  uint64_t tk = kPadKey;
+  for (int i0 = 0; i0 < m; i0 += kWave) {
+    uint64_t key = kPadKey;
+    if (i0 + lane < m) {
+      key = list[q * cap + i0 + lane];
+      if constexpr (kFloat) {
+        typedef float gt_f4u __attribute__((ext_vector_type(4), aligned(4)));
+        const float* const x = reinterpret_cast<const float*>(base + (int64_t)key * row_bytes);
+        float s = 0.f;
+        int i = 0;
+        for (; i + 4 <= dim; i += 4) {
+          const gt_f4u v = *reinterpret_cast<const gt_f4u*>(x + i);
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float d = qs[wave][i + e] - v[e];
+            s = __fmaf_rn(d, d, s);
+          }
+        }
+        for (; i < dim; i++) {
+          const float d = qs[wave][i] - x[i];
+          s = __fmaf_rn(d, d, s);
+        }
+        key |= (uint64_t)__float_as_uint(s) << 32;
+      }
+    }
+    // the first 64 sorted at once, the others offered one by one
+    if (i0 == 0) {
+      tk = ~wave_sort_desc(~key);
+      if (lane >= k) tk = kPadKey;
+    } else {
+      gt_offer(tk, k, key);
+    }
+  }
+  if (last) {
+    if (lane < k) {
+      ids[q * k + lane] = tk == kPadKey ? -1 : (int32_t)(uint32_t)tk;
+      dists[q * k + lane] = tk == kPadKey ? __int_as_float(0x7f800000) : __uint_as_float((uint32_t)(tk >> 32));
+    }
+    return;
+  }
+  // the k found so far open the next level's list
+  const uint64_t have = __ballot(lane < k && tk != kPadKey);
+  if (lane < k && tk != kPadKey) list[q * cap + lane] = kFloat ? (uint64_t)(uint32_t)tk : tk;
+  if (lane == k - 1) {
+    cnt[q] = (uint32_t)__popcll(have);
+    const float d = __uint_as_float((uint32_t)(tk >> 32));
+    if constexpr (kFloat) {
+      // a row is dropped when q.x (the bound) < ((1 - eps)(|q|^2 + |x|^2) - d) / 2;
+      // with no bound for the query (norm or distance not finite) none is
+      const float n2 = __uint_as_float(qn[q]);
+      const double at = 0.5 * ((1.0 - (double)kGtEps) * (double)n2 - (double)d) - 1e-30;
+      thr[q] = __float_as_uint(tk != kPadKey && n2 <= kGtHuge && d <= kGtHuge ? __double2float_rd(at)
+                                                                              : -__int_as_float(0x7f800000));
+    } else {
+      // dist = |q|^2 - 2 sum - (|x|^2 & 1) <= d needs sum >= (|q|^2 - d - 1) / 2
+      tkey[q] = tk;
+      thr[q] = (uint32_t)(tk != kPadKey ? ((int32_t)qn[q] - (int32_t)d) >> 1 : INT32_MIN);
+    }
+  }
+}
+
 int grid_of(int64_t work, int block) {
   return (int)std::max<int64_t>(1, std::min<int64_t>((work + block - 1) / block, 1 << 20));
 }
 
+// The scan of one batch of queries, all levels (see above).
+template <class T, int KS, int QT>
+void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
+               float* d_dists, int cap, int64_t resident, uint8_t* work, int32_t* d_lost, hipStream_t st) {
+  const int64_t groups = (nq + 128 * QT - 1) / (128 * QT), padded = groups * 128 * QT;
+  uint64_t* const list = reinterpret_cast<uint64_t*>(work);
+  uint64_t* const tkey = list + nq * cap;
+  uint32_t* const qn = reinterpret_cast<uint32_t*>(tkey + padded);
+  uint32_t* const thr = qn + padded;
+  uint32_t* const cnt = thr + padded;
+  uint8_t* const qp = reinterpret_cast<uint8_t*>(cnt + padded);
+  hipLaunchKernelGGL((gt_pack_kernel<T, KS>), dim3((unsigned)padded), dim3(64), 0, st, d_q, nq, dim, qp, qn, thr, tkey,
+                     cnt, d_lost);
+  HIP_OK(hipGetLastError());
+  ScanArgs a{};
+  a.base = reinterpret_cast<const uint8_t*>(d_base);
+  a.row_bytes = (int64_t)dim * (int64_t)sizeof(T);
+  a.nq = nq;
+  a.groups = (int)groups;
+  a.qp = qp;
+  a.qn = qn;
+  a.thr = thr;
+  a.tkey = tkey;
+  a.cnt = cnt;
+  a.list = list;
+  a.cap = cap;
+  a.over = d_lost;
+  int levels = 1;  // S = 4^(levels - 1): level 0 keeps all of its rows, at least k where n allows
+  a.period = 1;
+  while (n / (4 * a.period) >= (k <= 16 ? 64 : 256)) {
+    a.period *= 4;
+    levels++;
+  }
+  for (int l = 0; l < levels; l++) {
+    const int64_t w = l == 0 ? 1 : (int64_t)1 << (2 * (l - 1)), width = l == 0 ? 1 : 3 * w;
+    a.shift = l == 0 ? -1 : 2 * (l - 1);
+    a.rows = n / a.period * width +
+             std::max<int64_t>(0, std::min<int64_t>(n % a.period - (l == 0 ? 0 : w), width));
+    const int64_t tiles = (a.rows + kGtRows - 1) / kGtRows;
+    // as many workgroups as are resident at once, in eighths (one per XCD)
+    a.slices = (int)(8 * std::max<int64_t>(1, std::min<int64_t>((tiles + 7) / 8, resident / (8 * groups))));
+    hipLaunchKernelGGL((gt_scan_kernel<T, KS, QT>), dim3((unsigned)(groups * a.slices)), dim3(256),
+                       (size_t)gt_scan_lds<T>(KS, QT), st, a);
+    HIP_OK(hipGetLastError());
+    hipLaunchKernelGGL(gt_pick_kernel<T>, dim3((unsigned)((nq + 3) / 4)), dim3(256), 0, st, a.base, a.row_bytes, dim,
+                       d_q, nq, k, qn, thr, tkey, cnt, list, cap, l == levels - 1, d_ids, d_dists);
+    HIP_OK(hipGetLastError());
+  }
+}
+
+template <class T, int KS, int QT>
+bool gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
+                  float* d_dists, int device, hipStream_t st) {
+  const void* const fn = reinterpret_cast<const void*>(&gt_scan_kernel<T, KS, QT>);
+  HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, gt_scan_lds<T>(KS, QT)));
+  int per_cu = 0, cus = 0;
+  HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, (size_t)gt_scan_lds<T>(KS, QT)));
+  HIP_OK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  const int cap = k <= 16 ? 512 : 2048;  // level 0 keeps up to 256 (1024) rows, a later one about 3 k
+  const int64_t batch = std::min<int64_t>(nq, kGtBatch);
+  const int64_t padded = (batch + 128 * QT - 1) / (128 * QT) * (128 * QT);
+  const size_t bytes = (size_t)batch * cap * 8 + (size_t)padded * (8 + 12 + GtKind<T>::kPlanes * KS * 32) + 8;
+  uint8_t* work = nullptr;
+  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&work), bytes, st));
+  int32_t* const d_lost = reinterpret_cast<int32_t*>(work + bytes - 8);
+  HIP_OK(hipMemsetAsync(d_lost, 0, 8, st));
+  for (int64_t q = 0; q < nq; q += batch)
+    gt_levels<T, KS, QT>(d_base, n, dim, d_q + q * dim, std::min(batch, nq - q), k, d_ids + q * k, d_dists + q * k, cap,
+                         (int64_t)per_cu * cus, work, d_lost, st);
+  int32_t lost = 0;
+  HIP_OK(hipMemcpyAsync(&lost, d_lost, sizeof(lost), hipMemcpyDeviceToHost, st));
+  HIP_OK(hipFreeAsync(work, st));
+  HIP_OK(hipStreamSynchronize(st));
+  return lost == 0;
+}
+
+// The matrix-core path where it applies; false (results to be recomputed) for
+// rows longer than its tiles, 8-bit queries that are no whole numbers of the
+// element type, or an overflowed candidate list.
+template <class T>
+bool gt_matrix(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
+               float* d_dists, int device, hipStream_t st) {
+  const bool few = nq <= 256;  // one query tile per wave: a workgroup then holds 128 queries, not 256 or 512
+#define QV_GT(KS, QT) return gt_matrix_ks<T, KS, QT>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, st)
+  if constexpr (sizeof(T) == 4) {
+    if (dim > 128) return false;
+    if (few) {
+      if (dim <= 32) QV_GT(2, 1);
+      if (dim <= 64) QV_GT(4, 1);
+      if (dim <= 96) QV_GT(6, 1);
+      QV_GT(8, 1);
+    }
+    if (dim <= 32) QV_GT(2, 2);
+    if (dim <= 64) QV_GT(4, 2);
+    if (dim <= 96) QV_GT(6, 2);
+    QV_GT(8, 2);
+  } else {
+    if (dim > 256) return false;
+    if (few) {
+      if (dim <= 64) QV_GT(2, 1);
+      if (dim <= 128) QV_GT(4, 1);
+      QV_GT(8, 1);
+    }
+    if (dim <= 64) QV_GT(2, 4);
+    if (dim <= 128) QV_GT(4, 4);
+    QV_GT(8, 2);
+  }
+#undef QV_GT
+}
+
 template <class T>
 void ground_truth_t(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
-                    float* d_dists, hipStream_t st) {
+                    float* d_dists, int device, hipStream_t st) {
+  if (gt_matrix<T>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, st)) return;
   if constexpr (sizeof(T) == 1) {
     if (dim <= 4 * kGtWords && dim % 4 == 0 && k <= kGtMaxK) {
       int32_t* d_bad = nullptr;
@@ -319,11 +971,11 @@ int qv_ground_truth(const void* d_base, int32_t data_type, int64_t n, int32_t di
     hipStream_t st;
     HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     if (data_type == QV_UINT8)
-      ground_truth_t<uint8_t>(static_cast<const uint8_t*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, st);
+      ground_truth_t<uint8_t>(static_cast<const uint8_t*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, device, st);
     else if (data_type == QV_INT8)
-      ground_truth_t<int8_t>(static_cast<const int8_t*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, st);
+      ground_truth_t<int8_t>(static_cast<const int8_t*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, device, st);
     else
-      ground_truth_t<float>(static_cast<const float*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, st);
+      ground_truth_t<float>(static_cast<const float*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, device, st);
     HIP_OK(hipStreamDestroy(st));
   });
 }
