@@ -55,7 +55,7 @@ extern "C" {
                                      query the call can have in flight (min(nq,
                                      num_blocks x queries_per_block)), else shared
                                      pivots where the index allows them */
-#define QV_KERNEL_LUT 1           /* per-query fp32 LUT in LDS, one wave per workgroup */
+#define QV_KERNEL_LUT 1           /* per-query fp32 LUT in LDS, one workgroup per query */
 #define QV_KERNEL_SHARED_PIVOTS 2 /* PQ pivots once per CU in LDS, each LUT entry
                                      recomputed where it is read; needs chunks of
                                      4 dims (M = 32) or 2 dims (M = 48) */

@@ -238,12 +238,14 @@ __device__ __forceinline__ uint64_t wave_min_key(uint64_t key, bool valid, int* 
 // (chunk, pivot) cell accumulates its dimensions in ascending order, exactly as
 // the reference's i-ordered loop does; the fused multiply-add matches nvcc's
 // contraction of `dist_vec[..] += dist * dist`.  Lane l owns pivots 4l..4l+3.
+// Chunks first, first + step, ... (waves that share a table take turns).
 __device__ __forceinline__ void build_lut_lds(const float* __restrict__ qc_lds,
                                               const float* __restrict__ pivots_t,
                                               const int32_t* __restrict__ chunk_off,
-                                              int num_chunks, float* __restrict__ lut) {
+                                              int num_chunks, float* __restrict__ lut, int first = 0,
+                                              int step = 1) {
   const int lane = lane_id();
-  for (int m = 0; m < num_chunks; m++) {
+  for (int m = first; m < num_chunks; m += step) {
     const int o0 = chunk_off[m], o1 = chunk_off[m + 1];
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int i = o0; i < o1; i++) {

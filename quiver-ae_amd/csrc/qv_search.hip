@@ -3,10 +3,13 @@
 // Reference path (ruc-system/quiver-ae): persistent_search_kernel
 // (src/quiver/kernel_core/kernel_q1.cuh:20-757) driven by run_persistent_search
 // (src/quiver/search.cu:357-1361).  Differences by design:
-//   * one 64-lane wavefront per query, in one of two kernels: search_kernel
-//     (one-wave workgroups, the query's fp32 LUT in LDS) or search_kernel_sp
-//     (one workgroup of up to 16 waves per CU sharing the PQ pivots in LDS,
-//     each LUT entry recomputed where it is read); query and beam live in LDS;
+//   * one 64-lane wavefront owns a query's beam, in one of two kinds of kernel:
+//     with the query's fp32 LUT in LDS (search_kernel_team, a workgroup of
+//     three waves, two of them reading nodes and summing distances ahead;
+//     search_kernel, one wave, for the sizes the team does not take) or
+//     search_kernel_sp (one workgroup of up to 16 waves per CU sharing the PQ
+//     pivots in LDS, each LUT entry recomputed where it is read); query and
+//     beam live in LDS;
 //     neighbour lists, vectors and PQ codes are read straight from HBM (no CPU
 //     poll threads, no 4 KB page copies), and the next node's record is
 //     requested while the current hop finishes;
@@ -126,8 +129,8 @@ __global__ __launch_bounds__(256) void neighbour_codes_kernel(const uint8_t* pag
 // qv_search_r128.hip and qv_search_deep.hip.
 template <class T, int Q>
 KernelFn pick_mc(int M) {
-  if (M == 32) return search_kernel<T, Q, 32, 1>;
-  if (M == 48) return search_kernel<T, Q, 48, 1>;
+  if (M == 32) return search_kernel_team<T, Q, 32>;
+  if (M == 48) return search_kernel_team<T, Q, 48>;
   return search_kernel<T, Q, 0, 1>;
 }
 
@@ -219,6 +222,7 @@ struct LaunchPlan {
   int variant = QV_KERNEL_LUT;
   int lds_shared = 0;  // LDS of the workgroup beside its waves' (the shared pivots)
   int lds_wave = 0;    // LDS per wave (query)
+  int team = 1;        // waves per query (kTeamWaves: the team kernel)
 };
 
 // Grid of a launch holding `slots` query slots.  A shared-pivot workgroup
@@ -757,7 +761,7 @@ static int occupancy(int device, int lds_cu, KernelFn k, int waves, int lds) {
   return nb;
 }
 
-// The per-query-LUT kernel (one wave per workgroup, as many per CU as the LDS
+// The per-query-LUT kernel (one query per workgroup, as many per CU as the LDS
 // holds), or the shared-pivot kernel when the index has chunks of 4 dims
 // (M = 32) or 2 dims (M = 48), one workgroup of more waves fits a CU and more
 // than the LUT kernel's resident slots would be busy (`need`: queries the
@@ -780,8 +784,9 @@ LaunchPlan launch_plan(qv_index* ix, int ef, int want, int64_t need, int topk) {
                                : pick_kernel(ix->lay.data_type, P, M, npl));
   if (!lut.kern) fail(QV_EUNSUPPORTED, "no search kernel for this top-k, degree and ef");
   lut.waves = 1;
-  lut.lds = lds_plan(M, d, P, true, ef, topk).total;
-  lut.slots_per_cu = occupancy(ix->device, ix->lds_cu, lut.kern, 1, lut.lds);
+  lut.team = team_kernel(P, M, npl) ? kTeamWaves : 1;
+  lut.lds = lds_plan(M, d, P, true, ef, topk, lut.team > 1).total;
+  lut.slots_per_cu = occupancy(ix->device, ix->lds_cu, lut.kern, lut.team, lut.lds);
   if (want == QV_KERNEL_LUT) return lut;
   const bool forced = want == QV_KERNEL_SHARED_PIVOTS;
   if (wide) {
@@ -909,7 +914,7 @@ void search_record(qv_index* ix, const float* d_queries, int64_t nq, int ef, con
   a.rec_dists = rec.dists;
   a.rec_cap = rec.cap;
   HIP_OK(hipMemsetAsync(ix->d_counters, 0, 64, ix->stream));
-  hipLaunchKernelGGL(lp.kern, dim3(grid), dim3(kWave * ls.waves), (size_t)ls.lds, ix->stream, a);
+  hipLaunchKernelGGL(lp.kern, dim3(grid), dim3(kWave * ls.waves * lp.team), (size_t)ls.lds, ix->stream, a);
   HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(ix->stream));
   int32_t counters[4] = {0, 0, 0, 0};
@@ -1129,7 +1134,7 @@ void search(qv_index* ix, const float* queries, int64_t nq, int dim, int topk, i
     HIP_OK(hipMemcpyAsync(ix->d_queries, queries, sizeof(float) * (size_t)nq * dim, hipMemcpyHostToDevice,
                           ix->stream));
   HIP_OK(hipEventRecord(ix->ev0, ix->stream));
-  hipLaunchKernelGGL(lp.kern, dim3(grid), dim3(kWave * ls.waves), (size_t)ls.lds, ix->stream, a);
+  hipLaunchKernelGGL(lp.kern, dim3(grid), dim3(kWave * ls.waves * lp.team), (size_t)ls.lds, ix->stream, a);
   HIP_OK(hipGetLastError());
   HIP_OK(hipEventRecord(ix->ev1, ix->stream));
   // The launch counters follow the kernel into pinned memory on its stream, so
@@ -1460,7 +1465,7 @@ void search_noalloc(qv_index* ix, const float* d_queries, int64_t nq, int dim, i
 
   const auto t0 = std::chrono::steady_clock::now();
   HIP_OK(hipEventRecord(ix->ev0, ix->stream));
-  hipLaunchKernelGGL(lp.kern, dim3(ls.grid), dim3(kWave * ls.waves), (size_t)ls.lds, ix->stream, a);
+  hipLaunchKernelGGL(lp.kern, dim3(ls.grid), dim3(kWave * ls.waves * lp.team), (size_t)ls.lds, ix->stream, a);
   HIP_OK(hipGetLastError());
   HIP_OK(hipEventRecord(ix->ev1, ix->stream));
   unsigned long long* const totals = reinterpret_cast<unsigned long long*>(base + 64);

@@ -114,9 +114,23 @@ constexpr int kStageHead = 8;
 // (dim <= 32 kVecPre) its beam overlays both query copies, qc and qu, which
 // are only read once, into registers (load_query_dpp, load_query_pre),
 // before the first hop.
+__host__ __device__ inline int max_int(int x, int y) { return x > y ? x : y; }
+
 struct LdsPlan {
   int lut_off, qc_off, qu_off, beam_off, count_off, wide_off, total;
+  int slot_off, ctrl_off;  // team kernel: the evaluators' answers, the request words
 };
+
+// Team kernel: a query's workgroup is one wave that owns the beam and
+// kTeamEval evaluator waves that read nodes' records and code rows and sum
+// their neighbours' distances for it.
+constexpr int kTeamEval = 2;
+constexpr int kTeamWaves = 1 + kTeamEval;
+// LDS of one evaluator's answer: 64 keys, then the degree and the node's
+// exact distance.  The answers overlay the query copies where no wave reads
+// those after the LUT is built (dim <= 32 kVecPre).
+constexpr int kTeamSlot = kWave * 8 + 16;
+constexpr int kTeamCtrl = 48;  // [kTeamEval] request words, [kTeamEval] done words, the query id
 
 // Top-k entries a wave holds in its registers: entry i in lane i.  The
 // per-query-LUT kernel keeps entries 64 .. k - 1 of a larger k in LDS after
@@ -136,7 +150,8 @@ __host__ __device__ inline int beam_cap(int ef, int Q, bool lut) { return lut ? 
 // CU.  The other kernels add the candidates one at a time.
 __host__ __device__ constexpr bool rank_counts(bool lut, int Q) { return lut && Q <= 7; }
 
-__host__ __device__ inline LdsPlan lds_plan(int num_chunks, int dim, int Q, bool lut, int ef, int topk) {
+__host__ __device__ inline LdsPlan lds_plan(int num_chunks, int dim, int Q, bool lut, int ef, int topk,
+                                            bool team = false) {
   LdsPlan p;
   p.lut_off = 0;
   p.qc_off = p.lut_off + (lut ? num_chunks * kPivots * 4 : 0);
@@ -144,10 +159,19 @@ __host__ __device__ inline LdsPlan lds_plan(int num_chunks, int dim, int Q, bool
   p.qu_off = p.qc_off + dpad * 4;
   const bool overlay = !lut && dim <= 32 * kVecPre;
   p.beam_off = overlay ? p.qc_off : (p.qu_off + dpad * 4 + 15) & ~15;
+  p.slot_off = p.ctrl_off = 0;
+  if (team) {
+    p.slot_off = dim <= 32 * kVecPre ? p.qc_off : p.beam_off;
+    p.beam_off = max_int(p.beam_off, p.slot_off + kTeamEval * kTeamSlot);
+  }
   const int beam_bytes = beam_cap(ef, Q, lut) * 8;
   p.count_off = p.beam_off + beam_bytes;  // (rank_counts: no overlay)
   p.total = p.beam_off + (overlay && 2 * dpad * 4 > beam_bytes ? 2 * dpad * 4 : beam_bytes) +
             (rank_counts(lut, Q) ? beam_cap(ef, Q, lut) * 4 : 0);
+  if (team) {
+    p.ctrl_off = p.total;
+    p.total += kTeamCtrl;
+  }
   p.wide_off = p.total;
   if (lut) p.total += wide_topk(topk) * 8;
   return p;
@@ -169,6 +193,11 @@ constexpr int kXlQ = 32;
 // per lane and neighbour slots per lane: 16 (128 registers per wave), or 8
 // (256) for beams of more than 7 positions per lane and for two slots.
 __host__ __device__ constexpr int sp_max_waves(int Q, int NPL) { return Q <= 7 && NPL == 1 ? 16 : 8; }
+
+// Whether the per-query-LUT search of these sizes runs on the team kernel: one
+// neighbour slot per lane, code rows in registers, and a beam whose wave needs
+// no more than the registers three waves per SIMD leave (Q <= 7).
+__host__ __device__ inline bool team_kernel(int Q, int M, int npl) { return npl == 1 && Q <= 7 && (M == 32 || M == 48); }
 
 // Kernels instantiated in qv_search_r128.hip (two neighbour slots per lane,
 // Q rounded up to 1, 2, 4, 7, 10 or 16) and qv_search_deep.hip (one slot per
@@ -221,7 +250,7 @@ struct Taken {
 // shared pivots (chunks of SC dimensions).  NPL = 1: R <= 64, lane l owns
 // neighbour l; NPL = 2: R <= 128, lane l also owns neighbour l + 64.  WK: a
 // top-k above 64 (per-query LUT only), entries past the 64th in LDS.
-template <class T, int Q, int MC, int SC, int NPL, bool WK = false>
+template <class T, int Q, int MC, int SC, int NPL, bool WK = false, bool TM = false>
 struct Query {
   static_assert(NPL == 1 || NPL == 2, "one or two neighbours per lane");
   static_assert(!WK || SC == 0, "a top-k above 64 runs on the per-query-LUT kernel");
@@ -305,7 +334,7 @@ struct Query {
     for (int k = 0; k < Q; k++) ck[k] = kPadKey;
 #pragma unroll
     for (int j = 0; j < Q - 1; j++) pk[j] = kPadKey;
-    LdsPlan pl = lds_plan(a.num_chunks, a.dim, Q, SC == 0, a.ef, a.topk);
+    LdsPlan pl = lds_plan(a.num_chunks, a.dim, Q, SC == 0, a.ef, a.topk, TM);
     cap = beam_cap(a.ef, Q, SC == 0);
     wd = reinterpret_cast<float*>(smem + pl.wide_off);
     wi = reinterpret_cast<int32_t*>(wd + wide_topk(a.topk));
@@ -379,6 +408,10 @@ struct Query {
       e = exact_reduce(part, lane);
     else
       e = exact_l2_rest<T>(part, rec, qu, a.dim, lane);
+    insert_exact(v, e, lane);
+  }
+
+  __device__ __forceinline__ void insert_exact(int32_t v, float e, int lane) {
     last_e = e;
     if constexpr (WK) {
       wide_insert(e, v, lane);
@@ -579,6 +612,125 @@ struct Query {
     if constexpr (PF == 2 && kRows) have = nxt >= 0;
     if constexpr (PF != 0) take(nr, tk, lane);
     return nx;
+  }
+
+  // ---- team kernel: the beam's wave --------------------------------------
+  //
+  // One wave issues about 900 dependent instructions per hop and is alone on
+  // its SIMD in a small batch, so a hop takes 1.45 us even when everything it
+  // reads is in cache.  Here the evaluators take the loads, the ADC sums and
+  // the exact distance, and this wave the beam: it asks for a node (ask) as
+  // soon as it may be the next, so the two overlap.  Asking is only a guess:
+  // an answer is a function of the node and the query, and the beam takes an
+  // answer when its turn comes, so results do not depend on what was asked.
+  //
+  // A request is one 8-byte word, (number << 32) | node; the evaluator answers
+  // by writing its slot and then the same word to its done word.  Both sides'
+  // LDS accesses complete in order, so a reader that sees the done word sees
+  // the slot; a slot is asked again only after its last answer is not needed.
+  //
+  // Measured (1M x 128 uint8, ef = 208, pipe width 2): a hop 1.80 -> 1.45 us
+  // for one query, a call 414 -> 346 us; 16 queries of 96 floats in host
+  // buffers 340 -> 263 us; 3,000 top-100 queries over 1,024 teams 2.15 -> 1.72
+  // ms.  What is left of the hop, in cycles: 440 for the answer, 350 for the
+  // next request and the top-k, 950 for the ranks in the beam, 270 for the
+  // selection, 980 for the merge.
+  struct Team {
+    uint64_t* req;        // [kTeamEval]
+    uint64_t* done;       // [kTeamEval]
+    char* slot;           // [kTeamEval][kTeamSlot]
+    uint64_t word[kTeamEval];  // the last request of each evaluator
+    uint32_t number;
+  };
+  static constexpr int32_t kTeamQuit = -1;
+
+  static __device__ __forceinline__ void lds_put(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  static __device__ __forceinline__ uint64_t lds_get(const uint64_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+
+  // Asks evaluator e for v unless one of them has it.
+  __device__ __forceinline__ void ask(Team& tm, int e, int32_t v, int lane) const {
+    if ((int32_t)tm.word[0] == v || (int32_t)tm.word[1] == v) return;
+    tm.number++;
+    const uint64_t w = ((uint64_t)tm.number << 32) | (uint32_t)v;
+    if (e == 0)
+      tm.word[0] = w;
+    else
+      tm.word[1] = w;
+    if (lane == 0) lds_put(tm.req + e, w);
+  }
+
+  // hop of the team's beam wave: nxt is the expansion known to come next (-1:
+  // none), guess says whether the selection is expanded soon (pipe widths 1
+  // and 2).
+  __device__ __forceinline__ int32_t hop_team(int32_t v, Team& tm, int32_t nxt, bool guess) {
+    const int lane = opaque_lane();
+    ask(tm, (int32_t)tm.word[0] == nxt ? 1 : 0, v, lane);
+    const int at = (int32_t)tm.word[0] == v ? 0 : 1;
+    if (nxt >= 0) ask(tm, 1 - at, nxt, lane);
+    const uint64_t want = at == 0 ? tm.word[0] : tm.word[1];
+    const char* const slot = tm.slot + at * kTeamSlot;
+    uint64_t nkey, info;
+    // (bounded: an evaluator answers every request; the limit only keeps a
+    // broken launch from spinning, and fails the search)
+    for (uint32_t n = 0;; n++) {
+      const uint64_t d = read_lane_u64(lds_get(tm.done + at), 0);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      nkey = reinterpret_cast<const uint64_t*>(slot)[lane];
+      info = *reinterpret_cast<const uint64_t*>(slot + kWave * 8);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      if (d == want) break;
+      if (n > (1u << 22)) {
+        if (lane == 0) atomicOr(&a.counters[2], kErrSpinTimeout);
+        break;
+      }
+    }
+    const int deg = read_lane_i32((int)(uint32_t)info, 0);
+    evals += deg;
+    // v's answer is taken: its evaluator gets the guess, the beam's first
+    // unvisited entry (which the selection is unless a candidate beats it).  A
+    // wrong guess leaves that evaluator busy: the selection then goes to the
+    // other one if that does not hold the next expansion.
+    if (guess && u < sz) ask(tm, at, (int32_t)key_id(bu), lane);
+    insert_exact(v, __uint_as_float(read_lane_u32((uint32_t)(info >> 32), 0)), lane);
+    bool hit = false;
+    Rec none;
+    return merge_select<true, false>(nkey, lane < deg, lane, none, false, bu, hit, nullptr, [&](int32_t id) {
+      if (guess) ask(tm, nxt >= 0 ? at : 1 - at, id, lane);
+    });
+  }
+
+  // An evaluator's share of a query: answers until the beam wave's quit.
+  __device__ __forceinline__ void answer(uint64_t* req, uint64_t* done, char* slot, uint64_t& seen) {
+    const int lane = opaque_lane();
+    Rec nr;
+    Tk tk;
+    CodeRow<MC> cr;
+    while (true) {
+      const uint64_t w = read_lane_u64(lds_get(req), 0);
+      if (w == seen) {
+        __builtin_amdgcn_s_sleep(1);
+        continue;
+      }
+      seen = w;
+      const int32_t v = (int32_t)w;
+      if (v == kTeamQuit) return;
+      fetch(v, lane, nr);
+      if (a.nbr_codes != nullptr) adc_load<MC>(cr, block(v), off_blk);
+      take(nr, tk, lane);
+      if (a.nbr_codes == nullptr) adc_load<MC>(cr, a.codes, tk.nbr[0]);
+      const uint8_t* rec = a.dim > 32 * kVecPre ? record(v) : nullptr;
+      const float e = exact_l2_rest<T>(tk.part, rec, qu, a.dim, lane);
+      const float d = adc_sum_at0<MC>(cr);
+      reinterpret_cast<uint64_t*>(slot)[lane] = lane < tk.deg ? make_key(d, tk.nbr[0], false) : sentinel_key(lane);
+      if (lane == 0)
+        *reinterpret_cast<uint64_t*>(slot + kWave * 8) = ((uint64_t)__float_as_uint(e) << 32) | (uint32_t)tk.deg;
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      if (lane == 0) lds_put(done, w);
+    }
   }
 
   // hop with two neighbours per lane (R <= 128): the same expansion with the
@@ -801,9 +953,14 @@ struct Query {
   // hit: (PF) the selected node is the guessed one (key spec_key), whose
   // record the hop requested at its start.  SEL = false merges without a
   // selection (the first batch of a two-slot hop) and returns -1.
-  template <bool SEL, bool PF, bool ROWS = false>
+  // chosen(id): called with the selected node as soon as it is known.
+  struct NoHook {
+    __device__ __forceinline__ void operator()(int32_t) const {}
+  };
+  template <bool SEL, bool PF, bool ROWS = false, class Hook = NoHook>
   __device__ __forceinline__ int32_t merge_select(uint64_t nkey, bool has, int lane, Rec& nr, bool spec,
-                                                  uint64_t spec_key, bool& hit, CodeRow<MC>* cr = nullptr) {
+                                                  uint64_t spec_key, bool& hit, CodeRow<MC>* cr = nullptr,
+                                                  Hook chosen = Hook()) {
     const int ef = a.ef;
     // Candidates at or above the last entry of a full beam end beyond ef
     // (lastk: read with the previous merge's register reload).
@@ -917,6 +1074,7 @@ struct Query {
         selkey = kv0;
       }
     }
+    chosen((int32_t)key_id(selkey));
     if constexpr (PF) {
       // (the key test, not the position: a winning candidate lands at u too)
       hit = spec && selkey == spec_key;
@@ -1125,11 +1283,52 @@ __device__ __forceinline__ void query_sync() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 }
 
+// Team kernel, every wave of the workgroup: the query into LDS, this wave's
+// chunks of the LUT, this lane's query elements.  The answers' slots and the
+// beam may be written once the last barrier is passed.
+template <class Qu>
+__device__ __forceinline__ void team_query(const SearchArgs& a, Qu& Qy, const float* q) {
+  for (int i = (int)threadIdx.x; i < a.dim; i += kTeamWaves * kWave) {
+    const float c = query_elem(q, i) - a.centroid[i];
+    Qy.qc[i] = c;
+    Qy.qu[i] = c + a.centroid[i];
+  }
+  __syncthreads();
+  load_query_pre(Qy.qu, a.dim, lane_id(), Qy.quv);
+  build_lut_lds(Qy.qc, a.pivots_t, a.chunk_off, a.num_chunks, Qy.lut, (int)(threadIdx.x / kWave), kTeamWaves);
+  __syncthreads();
+}
+
 // The persistent query loop of one wave: smem is its LDS area, piv the
 // shared pivots (SC > 0).
-template <class T, int Q, int MC, int SC, int NPL, bool WK = false>
+template <class T, int Q, int MC, int SC, int NPL, bool WK = false, bool TM = false>
 __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, const float* piv) {
+  using Qu = Query<T, Q, MC, SC, NPL, WK, TM>;
   const int lane = lane_id();
+  // Team kernel: the evaluators loop here; the beam's wave (0) goes on below.
+  typename Qu::Team team;
+  int32_t* team_qid = nullptr;
+  if constexpr (TM) {
+    const LdsPlan pl = lds_plan(a.num_chunks, a.dim, Q, true, a.ef, a.topk, true);
+    team.req = reinterpret_cast<uint64_t*>(smem + pl.ctrl_off);
+    team.done = team.req + kTeamEval;
+    team.slot = smem + pl.slot_off;
+    team_qid = reinterpret_cast<int32_t*>(team.done + kTeamEval);
+    team.number = 0;
+    const int wave = (int)(threadIdx.x / kWave);
+    if (threadIdx.x < 2 * kTeamEval) team.req[threadIdx.x] = 0;  // ordered by the first barrier below
+    if (wave > 0) {
+      uint64_t seen = 0;
+      while (true) {
+        __syncthreads();  // the query's number is out
+        const int32_t qid = *team_qid;
+        if (qid < 0) return;
+        Qu Qy(a, smem, piv);
+        team_query(a, Qy, a.queries + (int64_t)qid * a.dim);
+        Qy.answer(team.req + wave - 1, team.done + wave - 1, team.slot + (wave - 1) * kTeamSlot, seen);
+      }
+    }
+  }
 
   while (true) {
     // ---- acquire (StreamingDispatch, src/quiver/kernel_core/policies/dispatch.cuh:39-79)
@@ -1190,6 +1389,10 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     if (pub != 0)
       __hip_atomic_fetch_max(a.feed_mirror + (int64_t)opaque_lane() * kFeedStride, pub, __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (TM) {
+      if (lane == 0) *team_qid = qid;
+      __syncthreads();
+    }
     if (qid < 0) break;
     // Later tickets issue first: the last-admitted queries set the end of the
     // launch, the earlier ones have time to spare.
@@ -1201,7 +1404,7 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     }
     if (a.t_start && lane == 0) a.t_start[qid] = wall_ticks();
 
-    Query<T, Q, MC, SC, NPL, WK> Qy(a, smem, piv);
+    Qu Qy(a, smem, piv);
     const float* q = a.queries + (int64_t)qid * a.dim;
     // ---- entry node: the nav-graph search on the raw query when a nav graph is
     // loaded (kernel_q1.cuh:148-174, 199-206), else the medoid.
@@ -1210,6 +1413,11 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
                                      : a.medoid;
     // ---- query into LDS: q - mu for the LUT, fl(fl(q - mu) + mu) for the exact
     // distance (pq_device.cuh:18-20, 33-35).
+    if constexpr (TM) {
+      team_query(a, Qy, q);
+#pragma unroll
+      for (int w = 0; w < kTeamEval; w++) team.word[w] = (uint64_t)(uint32_t)Qu::kTeamQuit;
+    } else {
     for (int i = lane; i < a.dim; i += kWave) {
       const float c = query_elem(q, i) - a.centroid[i];
       Qy.qc[i] = c;
@@ -1222,6 +1430,7 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     }
     load_query_pre(Qy.qu, a.dim, lane, Qy.quv);
     if constexpr (SC > 0) load_query_dpp(Qy.qc, a.dim, lane, Qy.qd);
+    }
     // qc and qu may share their LDS with the beam (lds_plan): no beam store
     // may move above these reads.
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1285,7 +1494,7 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     // holds.  (The address goes through an opaque lane value so the load is a
     // vector one: a scalar load's wait would also wait for the LDS traffic.
     // Also reading the ticket counter here measured up to a fifth slower.)
-    constexpr bool kTail = Query<T, Q, MC, SC, NPL>::kTail;
+    constexpr bool kTail = Qu::kTail;
     int32_t probe_w = 0, probe_at = 32;
     bool probing = false;
     auto tail_probe = [&]() -> bool {
@@ -1312,6 +1521,7 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     // v's; pf is the node so requested, fetched again when the guess was wrong.
     int32_t pf = -1;
     auto expand = [&](int32_t v, int32_t nxt, auto tl) -> int32_t {
+      if constexpr (TM) return Qy.hop_team(v, team, nxt, a.pipe_w <= 2);
       if (v != pf) {
         Qy.fetch(v, lane, nr);
         Qy.take(nr, tk, lane);
@@ -1326,14 +1536,20 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
       // One pipe lane (kernel_q1.cuh:199-397 boot, then 407-670): the node a
       // hop selects is the next one expanded, so its record is requested while
       // the hop finishes.
-      Qy.fetch(entry, lane, nr);
-      Qy.take(nr, tk, lane);
+      if constexpr (!TM) {
+        Qy.fetch(entry, lane, nr);
+        Qy.take(nr, tk, lane);
+      }
       int32_t v = entry;
       // true: go on from v in tail mode
       auto w1_loop = [&](auto tl) -> bool {
         constexpr bool TL = decltype(tl)::value;
         while (true) {
-          const int32_t nx = Qy.template hop<1, TL>(v, tk, nr, cr, have);
+          int32_t nx;
+          if constexpr (TM)
+            nx = Qy.hop_team(v, team, -1, true);
+          else
+            nx = Qy.template hop<1, TL>(v, tk, nr, cr, have);
           log_hop(v);
           ++step;
           bool to_tail = false;
@@ -1425,6 +1641,11 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     }
 
   finish:
+    if constexpr (TM) {
+      // the evaluators go to the next query's barrier
+      team.number++;
+      if (lane < kTeamEval) Qu::lds_put(team.req + lane, ((uint64_t)team.number << 32) | (uint32_t)Qu::kTeamQuit);
+    }
     // ---- finish (kernel_q1.cuh:662-704)
     if (sr) {
       if (sr_at < 0) sr_h = sr_hits();
@@ -1452,12 +1673,12 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
         __hip_atomic_store(&a.ring[pos], qid + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
-    query_sync<SC>();
+    if constexpr (!TM) query_sync<SC>();
   }
   // This wave has no more queries: one more ended wave of its workgroup (the
   // tail-mode probe of the others reads it).  Release at workgroup scope: the
   // count is published after this wave's last pivot reads are done.
-  if constexpr (Query<T, Q, MC, SC, NPL>::kTail) {
+  if constexpr (Qu::kTail) {
     if (a.wg_done && lane == 0)
       __hip_atomic_fetch_add(a.wg_done + blockIdx.x, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
@@ -1469,6 +1690,13 @@ template <class T, int Q, int MC, int NPL, bool WK = false>
 __global__ __launch_bounds__(64) void search_kernel(SearchArgs a) {
   extern __shared__ __align__(16) char smem[];
   run_queries<T, Q, MC, 0, NPL, WK>(a, smem, nullptr);
+}
+
+// One query per workgroup of kTeamWaves waves (the team kernel).
+template <class T, int Q, int MC, bool WK = false>
+__global__ __launch_bounds__(kTeamWaves * 64) void search_kernel_team(SearchArgs a) {
+  extern __shared__ __align__(16) char smem[];
+  run_queries<T, Q, MC, 0, 1, WK, true>(a, smem, nullptr);
 }
 
 // One workgroup per CU, one query per wave: the workgroup holds the pivots

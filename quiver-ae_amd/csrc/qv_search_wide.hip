@@ -11,8 +11,13 @@ namespace {
 
 template <class T, int Q, int NPL>
 KernelFn wide_mc(int M) {
-  if (M == 32) return search_kernel<T, Q, 32, NPL, true>;
-  if (M == 48) return search_kernel<T, Q, 48, NPL, true>;
+  if constexpr (NPL == 1 && Q <= 7) {
+    if (M == 32) return search_kernel_team<T, Q, 32, true>;
+    if (M == 48) return search_kernel_team<T, Q, 48, true>;
+  } else {
+    if (M == 32) return search_kernel<T, Q, 32, NPL, true>;
+    if (M == 48) return search_kernel<T, Q, 48, NPL, true>;
+  }
   return search_kernel<T, Q, 0, NPL, true>;
 }
 
