@@ -9,10 +9,10 @@
 //   * Medoid: the point nearest to the mean of all points.
 //   * Graph: Vamana with batched insertion (batch sizes double up to a cap).  For
 //     each batch the persistent search kernel runs a beam search of width L for
-//     every inserted point and records the expanded nodes; a wave per point then
+//     every inserted point and records the expanded nodes; a workgroup per point then
 //     applies RobustPrune(alpha, R) to expanded nodes plus current neighbours;
 //     reverse edges are sorted by target (rocPRIM radix sort) and a wave per
-//     target merges them, pruning again when the list would exceed R.
+//     target merges them, a workgroup pruning again when the list would exceed R.
 // Every step is deterministic for a given seed.
 #include <cstring>
 
@@ -377,42 +377,10 @@ __global__ void init_pages_kernel(GLayout L, const T* __restrict__ base) {
   }
 }
 
-// ---- wave RobustPrune ------------------------------------------------------
+// ---- RobustPrune -----------------------------------------------------------
 
-constexpr int kSlots = 8;            // candidate slots per lane (512 keys)
-constexpr int kMaxCand = kSlots * kWave;
-
-template <int P>
-__device__ __forceinline__ void wave_sort_asc_full(uint64_t (&b)[P]) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int k = 2; k <= P * kWave; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= kWave) {
-        const int js = j / kWave;
-#pragma unroll
-        for (int s = 0; s < P; s++) {
-          const int t = s ^ js;
-          if (t > s) {
-            const bool up = ((s * kWave) & k) == 0;
-            const uint64_t lo = umin64(b[s], b[t]), hi = umax64(b[s], b[t]);
-            b[s] = up ? lo : hi;
-            b[t] = up ? hi : lo;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int s = 0; s < P; s++) {
-          const uint64_t other = shfl_xor64(b[s], j);
-          const bool up = ((s * kWave + lane) & k) == 0;
-          const bool lower = (lane & j) == 0;
-          b[s] = (lower == up) ? umin64(b[s], other) : umax64(b[s], other);
-        }
-      }
-    }
-  }
-}
+constexpr int kMaxCand = 512;        // candidates before dedupe
+constexpr int kPruneThreads = 256;   // one candidate each after it
 
 template <class T>
 __device__ __forceinline__ int32_t vec_norm(const uint32_t* a, int ds4) {
@@ -450,20 +418,24 @@ struct PruneArgs {
   int G;                     // lanes that fetch one row together (power of two, >= 4)
 };
 
-// LDS of one prune wave: keys [cmax] u64, norms [cmax] i32, the centre row and
-// cmax candidate rows at `stride` dwords (16-byte aligned), then the output list.
-// The candidate rows double as the fetch phase's (id, distance) table.
+// LDS of one prune: keys [cmax] u64, norms [cmax] i32, the centre row and cmax
+// candidate rows at `stride` dwords (16-byte aligned), the output list, then the
+// greedy loop's masks and the compaction's counts.  The candidate rows double
+// as the fetch phase's (id, distance) table and the sorted keys.  rule: the
+// bytes that decide cmax (build_gpu_t).
 struct PruneLds {
-  int norms_off, cvec_off, vecs_off, outl_off, total;
+  int norms_off, cvec_off, vecs_off, outl_off, masks_off, rule, total;
 };
 __host__ __device__ inline PruneLds prune_lds_plan(int cmax, int stride, int R) {
   PruneLds p;
   p.norms_off = 8 * cmax;
   p.cvec_off = (12 * cmax + 15) & ~15;
   p.vecs_off = p.cvec_off + 4 * stride;
-  const int vec_bytes = 4 * cmax * stride > 8 * kMaxCand ? 4 * cmax * stride : 8 * kMaxCand;
-  p.outl_off = p.vecs_off + vec_bytes;
-  p.total = p.outl_off + 4 * R;
+  const int rows = 4 * cmax * stride;
+  p.rule = p.vecs_off + (rows > 8 * kMaxCand ? rows : 8 * kMaxCand) + 4 * R;
+  p.outl_off = p.vecs_off + (rows > 16 * kMaxCand ? rows : 16 * kMaxCand);
+  p.masks_off = (p.outl_off + 4 * R + 7) & ~7;
+  p.total = p.masks_off + 2 * (kPruneThreads / kWave) * (8 + 4);
   return p;
 }
 
@@ -496,17 +468,20 @@ __device__ __forceinline__ V group_sum(V v, int G) {
   return v;
 }
 
-// Squared distance of two LDS rows read 16 bytes at a time (q4 pieces; words
-// past the row are zero in both).  Float: the same dimension order as a
-// sequential loop; 8-bit data: exact integers from the dot product and norms.
-template <class T>
-__device__ __forceinline__ float lds_row_dist(const uint32_t* a, const uint32_t* b, int q4, int32_t na, int32_t nb) {
+// Squared distance of LDS row a (q4 pieces of 16 bytes, the same for every
+// lane) and this lane's row, held in registers when KR pieces hold it (b), else
+// in LDS (bl).  Words past the row are zero in both.  Float: the dimension
+// order of a sequential loop; 8-bit data: exact integers from the dot product
+// and the norms.
+template <class T, int KR>
+__device__ __forceinline__ float row_dist(const uint32_t* a, const uint4 (&b)[KR > 0 ? KR : 1], const uint32_t* bl,
+                                          int q4, int32_t na, int32_t nb) {
   const uint4* a4 = reinterpret_cast<const uint4*>(a);
-  const uint4* b4 = reinterpret_cast<const uint4*>(b);
-  if constexpr (sizeof(T) == 4) {
-    float s = 0.f;
-    for (int q = 0; q < q4; q++) {
-      const uint4 x = a4[q], y = b4[q];
+  const uint4* b4 = reinterpret_cast<const uint4*>(bl);
+  float s = 0.f;
+  int32_t acc = 0;
+  auto add = [&](const uint4& x, const uint4& y) {
+    if constexpr (sizeof(T) == 4) {
       float d = __uint_as_float(x.x) - __uint_as_float(y.x);
       s = __fmaf_rn(d, d, s);
       d = __uint_as_float(x.y) - __uint_as_float(y.y);
@@ -515,243 +490,78 @@ __device__ __forceinline__ float lds_row_dist(const uint32_t* a, const uint32_t*
       s = __fmaf_rn(d, d, s);
       d = __uint_as_float(x.w) - __uint_as_float(y.w);
       s = __fmaf_rn(d, d, s);
-    }
-    return s;
-  } else if constexpr (std::is_signed<T>::value) {
-    int32_t acc = 0;
-    for (int q = 0; q < q4; q++) {
-      const uint4 x = a4[q], y = b4[q];
+    } else if constexpr (std::is_signed<T>::value) {
       acc = __builtin_amdgcn_sdot4((int)x.x, (int)y.x, acc, false);
       acc = __builtin_amdgcn_sdot4((int)x.y, (int)y.y, acc, false);
       acc = __builtin_amdgcn_sdot4((int)x.z, (int)y.z, acc, false);
       acc = __builtin_amdgcn_sdot4((int)x.w, (int)y.w, acc, false);
+    } else {
+      acc = (int32_t)__builtin_amdgcn_udot4(x.x, y.x, (uint32_t)acc, false);
+      acc = (int32_t)__builtin_amdgcn_udot4(x.y, y.y, (uint32_t)acc, false);
+      acc = (int32_t)__builtin_amdgcn_udot4(x.z, y.z, (uint32_t)acc, false);
+      acc = (int32_t)__builtin_amdgcn_udot4(x.w, y.w, (uint32_t)acc, false);
     }
-    return (float)(na + nb - 2 * acc);
+  };
+  if constexpr (KR > 0) {
+#pragma unroll
+    for (int q = 0; q < KR; q++)
+      if (q < q4) add(a4[q], b[q]);
   } else {
-    uint32_t acc = 0;
-    for (int q = 0; q < q4; q++) {
-      const uint4 x = a4[q], y = b4[q];
-      acc = __builtin_amdgcn_udot4(x.x, y.x, acc, false);
-      acc = __builtin_amdgcn_udot4(x.y, y.y, acc, false);
-      acc = __builtin_amdgcn_udot4(x.z, y.z, acc, false);
-      acc = __builtin_amdgcn_udot4(x.w, y.w, acc, false);
-    }
-    return (float)((int64_t)na + (int64_t)nb - 2 * (int64_t)acc);
+    for (int q = 0; q < q4; q++) add(a4[q], b4[q]);
   }
+  if constexpr (sizeof(T) == 4) return s;
+  // (64-bit: rows of more than 32,768 bytes do not exist, sums of 8-bit squares fit 32)
+  else return (float)((int64_t)na + (int64_t)nb - 2 * (int64_t)acc);
 }
 
-// LDS areas of a prune wave.
-struct PruneSmem {
-  uint64_t* keys;
-  int32_t* norms;
-  uint32_t* cvec;
-  uint32_t* vecs;
-  uint32_t* outl;
-};
-
-// Prune of one centre over its C0 candidates (cand(i) -> node id, or -1 to
-// skip): exact distances from the centre, sort by (distance, id), dedupe, then
+// One workgroup of four waves per centre: forward prunes (mode 0: the nodes
+// expanded by the centre's build search, then its current list and pending
+// edges), reverse prunes of marked segments (mode 1: current list, pending
+// edges, then the segment's incoming sources) and the flush of pending edges
+// (mode 2: list and pending).  Per centre: exact distances to the candidates
+// (candidate i -> node id, or -1 to skip), sort by (distance, id), dedupe, then
 // the list is the candidates themselves when they fit in R, else
-// RobustPrune(alpha, R) over them.  SL slots of 64 lanes hold the sort
-// (C0 <= 64 SL).  The centre's pending edges are cleared: the caller put them
-// among the candidates.
-// Candidate rows are fetched cooperatively: G lanes per row, lane p of a row
-// reading words p, p + G, ... (a contiguous G-word run per load instruction),
-// 64 / G rows per instruction and two instructions' rows in flight, so the
-// fetch costs a few memory round trips per centre instead of one per word.
-template <class T, int SL, class F>
-__device__ __forceinline__ void prune_one(const PruneArgs& a, const PruneSmem& m, int64_t center, int C0, F cand) {
+// RobustPrune(alpha, R) over them.  The centre's pending edges are cleared: they
+// are among the candidates.
+//   * Candidate rows are fetched cooperatively: G lanes per row, lane p of a row
+//     reading words p, p + G, ... (a contiguous G-word run per load
+//     instruction), 64 / G rows per instruction and two instructions' rows in
+//     flight per wave.
+//   * Sorted by rank: a thread counts the keys below its own; equal keys are
+//     one node listed twice and share a place, whose gap the compaction closes.
+//   * A thread owns a candidate (cmax <= 256), its row in registers where KR
+//     16-byte pieces hold it: an accepted row is read from LDS by every lane at
+//     once, so a step of the greedy loop is one row of arithmetic and a barrier.
+// What bounds it: the candidate rows in LDS (37 KB of 128-byte rows, 74 KB of
+// 96 floats) allow four or two centres per CU, which with one wave per centre
+// left the SIMDs at one or half a wave each, waiting on LDS and on each row's
+// chain.  All prunes of a build of 250,000 x 128 uint8 (R = 64, L = 100): 84 ms
+// with one wave per centre, 40 ms; 100,003 x 96 float: 150 and 63 ms.
+template <class T, int KR>
+__global__ __launch_bounds__(kPruneThreads) void prune_kernel(PruneArgs a) {
   using Acc = RowAcc<T>;
   using AccT = typename Acc::type;
-  const GLayout& L = a.L;
-  const int lane = lane_id();
-  const int ds4 = (int)(L.data_size / 4);
-  const int S = a.stride;
-  const int w4 = (ds4 + 3) & ~3;  // row words read by lds_row_dist (zero past ds4)
-  const int G = a.G, rpr = kWave / G, p = lane & (G - 1), sub = lane / G;
-  const int kk = (ds4 + G - 1) / G;  // words per lane per row
-  uint32_t* cand_id = m.vecs;            // fetch phase: [kMaxCand] ids (~0u: none)
-  uint32_t* cand_d = m.vecs + kMaxCand;  // fetch phase: [kMaxCand] distance bits
-  uint32_t* crec = reinterpret_cast<uint32_t*>(node_rec(L, center));
-  uint32_t* cnb = crec + ds4;
-  const int32_t cnorm = vec_norm<T>(m.cvec, ds4);
-
-  // ---- distances centre -> candidates, rows fetched by groups of G lanes
-  for (int r0 = 0; r0 < C0; r0 += 2 * rpr) {
-    const int i0 = r0 + sub, i1 = r0 + rpr + sub;
-    const int64_t id0 = i0 < C0 ? cand(i0) : -1;
-    const int64_t id1 = i1 < C0 ? cand(i1) : -1;
-    const uint32_t* x0 = reinterpret_cast<const uint32_t*>(node_rec(L, id0 >= 0 ? id0 : center));
-    const uint32_t* x1 = reinterpret_cast<const uint32_t*>(node_rec(L, id1 >= 0 ? id1 : center));
-    AccT s0 = 0, s1 = 0;
-    for (int k0 = 0; k0 < kk; k0 += 4) {
-      uint32_t v0[4], v1[4], cw[4];
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int w = p + G * (k0 + t);
-        const bool ok = k0 + t < kk && w < ds4;
-        v0[t] = ok ? x0[w] : 0u;
-        v1[t] = ok ? x1[w] : 0u;
-        cw[t] = ok ? m.cvec[w] : 0u;
-      }
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        s0 = Acc::add(s0, cw[t], v0[t]);
-        s1 = Acc::add(s1, cw[t], v1[t]);
-      }
-    }
-    s0 = group_sum(s0, G);
-    s1 = group_sum(s1, G);
-    if (p == 0) {
-      float d0, d1;
-      if constexpr (sizeof(T) == 4) {
-        d0 = s0;
-        d1 = s1;
-      } else {
-        d0 = (float)(cnorm + s0);
-        d1 = (float)(cnorm + s1);
-      }
-      if (i0 < C0) {
-        cand_id[i0] = id0 >= 0 ? (uint32_t)id0 : ~0u;
-        cand_d[i0] = __float_as_uint(d0);
-      }
-      if (i1 < C0) {
-        cand_id[i1] = id1 >= 0 ? (uint32_t)id1 : ~0u;
-        cand_d[i1] = __float_as_uint(d1);
-      }
-    }
-  }
-  __syncthreads();
-  uint64_t b[SL];
-#pragma unroll
-  for (int s = 0; s < SL; s++) {
-    const int i = s * kWave + lane;
-    uint64_t key = kPadKey;
-    if (i < C0) {
-      const uint32_t id = cand_id[i];
-      if (id != ~0u) key = ((uint64_t)cand_d[i] << 32) | (uint64_t)id;
-    }
-    b[s] = key;
-  }
-  __syncthreads();  // the fetch table is overwritten by the rows below
-  wave_sort_asc_full<SL>(b);
-  // dedupe (equal ids are adjacent: equal distance) and compact into LDS
-  int C = 0;
-  uint32_t prev = 0xffffffffu;
-  bool prev_valid = false;
-#pragma unroll
-  for (int s = 0; s < SL; s++) {
-    const uint32_t id = (uint32_t)b[s];
-    uint32_t pid = (uint32_t)__shfl_up((int)id, 1);
-    bool pvalid = __shfl_up((int)(b[s] != kPadKey), 1) != 0;
-    if (lane == 0) {
-      pid = prev;
-      pvalid = prev_valid;
-    }
-    const bool keep = b[s] != kPadKey && !(pvalid && pid == id);
-    const uint64_t km = __ballot(keep);
-    const int pos = C + __popcll(km & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))));
-    if (keep && pos < a.cmax) m.keys[pos] = b[s];
-    C += __popcll(km);
-    prev = (uint32_t)__shfl((int)id, kWave - 1);
-    prev_valid = __shfl((int)(b[s] != kPadKey), kWave - 1) != 0;
-  }
-  C = min(C, a.cmax);
-  __syncthreads();
-
-  int out_n = 0;
-  if (C <= L.R) {
-    for (int i = lane; i < C; i += kWave) cnb[1 + i] = (uint32_t)m.keys[i];
-    out_n = C;
-  } else {
-    // stage the candidate rows (and their norms) in LDS, fetched as above
-    for (int r0 = 0; r0 < C; r0 += 2 * rpr) {
-      const int i0 = r0 + sub, i1 = r0 + rpr + sub;
-      const int64_t id0 = i0 < C ? (int64_t)(uint32_t)m.keys[i0] : center;
-      const int64_t id1 = i1 < C ? (int64_t)(uint32_t)m.keys[i1] : center;
-      const uint32_t* x0 = reinterpret_cast<const uint32_t*>(node_rec(L, id0));
-      const uint32_t* x1 = reinterpret_cast<const uint32_t*>(node_rec(L, id1));
-      AccT n0 = 0, n1 = 0;
-      for (int k0 = 0; k0 < kk; k0 += 4) {
-        uint32_t v0[4], v1[4];
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const int w = p + G * (k0 + t);
-          const bool ok = k0 + t < kk && w < ds4;
-          v0[t] = ok ? x0[w] : 0u;
-          v1[t] = ok ? x1[w] : 0u;
-        }
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const int w = p + G * (k0 + t);
-          if (k0 + t < kk && w < w4) {
-            if (i0 < C) m.vecs[i0 * S + w] = v0[t];
-            if (i1 < C) m.vecs[i1 * S + w] = v1[t];
-          }
-          n0 = Acc::norm_add(n0, v0[t]);
-          n1 = Acc::norm_add(n1, v1[t]);
-        }
-      }
-      if constexpr (sizeof(T) != 4) {
-        n0 = group_sum(n0, G);
-        n1 = group_sum(n1, G);
-        if (p == 0) {
-          if (i0 < C) m.norms[i0] = n0;
-          if (i1 < C) m.norms[i1] = n1;
-        }
-      }
-    }
-    __syncthreads();
-    uint32_t alive = 0;
-#pragma unroll
-    for (int s = 0; s < SL; s++)
-      if (s * kWave + lane < C) alive |= 1u << s;
-    const int q4 = w4 / 4;
-    for (int i = 0; i < C && out_n < L.R; i++) {
-      const uint32_t owner = (uint32_t)__shfl((int)alive, i & (kWave - 1));
-      if (!((owner >> (i >> 6)) & 1u)) continue;
-      if (lane == 0) m.outl[out_n] = (uint32_t)m.keys[i];
-      out_n++;
-      const uint32_t* vi = m.vecs + i * S;
-      const int32_t ni = sizeof(T) == 4 ? 0 : m.norms[i];
-#pragma unroll
-      for (int s = 0; s < SL; s++) {
-        const int j = s * kWave + lane;
-        if (j > i && j < C && ((alive >> s) & 1u)) {
-          const float dij = lds_row_dist<T>(vi, m.vecs + j * S, q4, ni, sizeof(T) == 4 ? 0 : m.norms[j]);
-          const float dpj = __uint_as_float((uint32_t)(m.keys[j] >> 32));
-          if (a.alpha * dij <= dpj) alive &= ~(1u << s);
-        }
-      }
-    }
-    __syncthreads();
-    for (int i = lane; i < out_n; i += kWave) cnb[1 + i] = m.outl[i];
-  }
-  if (lane == 0) {
-    cnb[0] = (uint32_t)out_n;
-    a.pcnt[center] = 0;
-  }
-  __syncthreads();
-}
-
-// One wave per centre: forward prunes (mode 0: the nodes expanded by the
-// centre's build search, then its current list and pending edges), reverse
-// prunes of marked segments (mode 1: current list, pending edges, then the
-// segment's incoming sources) and the flush of pending edges (mode 2: list and
-// pending).  The sort width follows the candidate count.
-template <class T>
-__global__ __launch_bounds__(64) void prune_kernel(PruneArgs a) {
   extern __shared__ __align__(16) char smem[];
   const GLayout& L = a.L;
-  const int lane = lane_id();
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  constexpr int kWaves = kPruneThreads / kWave;
   const int ds4 = (int)(L.data_size / 4);
   const PruneLds pl = prune_lds_plan(a.cmax, a.stride, L.R);
-  PruneSmem m;
-  m.keys = reinterpret_cast<uint64_t*>(smem);
-  m.norms = reinterpret_cast<int32_t*>(smem + pl.norms_off);
-  m.cvec = reinterpret_cast<uint32_t*>(smem + pl.cvec_off);
-  m.vecs = reinterpret_cast<uint32_t*>(smem + pl.vecs_off);
-  m.outl = reinterpret_cast<uint32_t*>(smem + pl.outl_off);
+  uint64_t* const keys = reinterpret_cast<uint64_t*>(smem);
+  int32_t* const norms = reinterpret_cast<int32_t*>(smem + pl.norms_off);
+  uint32_t* const cvec = reinterpret_cast<uint32_t*>(smem + pl.cvec_off);
+  uint32_t* const vecs = reinterpret_cast<uint32_t*>(smem + pl.vecs_off);
+  uint32_t* const outl = reinterpret_cast<uint32_t*>(smem + pl.outl_off);
+  uint64_t* const masks = reinterpret_cast<uint64_t*>(smem + pl.masks_off);  // [2][kWaves]
+  int32_t* const counts = reinterpret_cast<int32_t*>(masks + 2 * kWaves);    // [2 * kWaves]
+  // before the rows are staged, their place holds the fetch table and the sorted keys
+  uint32_t* const cand_id = vecs;             // [kMaxCand] ids (~0u: none)
+  uint32_t* const cand_d = vecs + kMaxCand;   // [kMaxCand] distance bits (~0u: none)
+  uint64_t* const sorted = reinterpret_cast<uint64_t*>(vecs + 2 * kMaxCand);  // [kMaxCand]
+  const int S = a.stride;
+  const int w4 = (ds4 + 3) & ~3;  // row words row_dist reads (zero past ds4)
+  const int G = a.G, rpr = kWave / G, p = lane & (G - 1), sub = lane / G;
+  const int kk = (ds4 + G - 1) / G;  // words per lane per row
   for (int64_t ci = blockIdx.x; ci < a.num_centers; ci += gridDim.x) {
     int64_t center;
     int64_t seg_begin = 0, seg_end = 0;
@@ -775,12 +585,12 @@ __global__ __launch_bounds__(64) void prune_kernel(PruneArgs a) {
         break;
       }
     }
-    uint32_t* crec = reinterpret_cast<uint32_t*>(node_rec(L, center));
-    for (int w = lane; w < a.stride; w += kWave) m.cvec[w] = w < ds4 ? crec[w] : 0u;
-    const uint32_t* cnb = crec + ds4;
+    uint32_t* const crec = reinterpret_cast<uint32_t*>(node_rec(L, center));
+    uint32_t* const cnb = crec + ds4;
+    for (int w = tid; w < a.stride; w += kPruneThreads) cvec[w] = w < ds4 ? crec[w] : 0u;
     const int cdeg = (int)cnb[0];
     const int pc = a.pcnt[center];
-    const uint32_t* pend = a.pend + center * a.P;
+    const uint32_t* const pend = a.pend + center * a.P;
     // candidate i: [lead candidates][current list][pending][trailing sources]
     int lead = 0, tail = 0;
     if (a.mode == 0) lead = min(a.hops[ci], a.rec_cap);
@@ -795,9 +605,180 @@ __global__ __launch_bounds__(64) void prune_kernel(PruneArgs a) {
       return id == center ? -1 : id;
     };
     __syncthreads();
-    if (C0 <= 2 * kWave) prune_one<T, 2>(a, m, center, C0, cand);
-    else if (C0 <= 4 * kWave) prune_one<T, 4>(a, m, center, C0, cand);
-    else prune_one<T, kSlots>(a, m, center, C0, cand);
+    const int32_t cnorm = vec_norm<T>(cvec, ds4);
+
+    // ---- distances centre -> candidates, rows fetched by groups of G lanes
+    for (int r0 = wave * 2 * rpr; r0 < C0; r0 += kWaves * 2 * rpr) {
+      const int i0 = r0 + sub, i1 = r0 + rpr + sub;
+      const int64_t id0 = i0 < C0 ? cand(i0) : -1;
+      const int64_t id1 = i1 < C0 ? cand(i1) : -1;
+      const uint32_t* x0 = reinterpret_cast<const uint32_t*>(node_rec(L, id0 >= 0 ? id0 : center));
+      const uint32_t* x1 = reinterpret_cast<const uint32_t*>(node_rec(L, id1 >= 0 ? id1 : center));
+      AccT s0 = 0, s1 = 0;
+      for (int k0 = 0; k0 < kk; k0 += 4) {
+        uint32_t v0[4], v1[4], cw[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const int w = p + G * (k0 + t);
+          const bool ok = k0 + t < kk && w < ds4;
+          v0[t] = ok ? x0[w] : 0u;
+          v1[t] = ok ? x1[w] : 0u;
+          cw[t] = ok ? cvec[w] : 0u;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          s0 = Acc::add(s0, cw[t], v0[t]);
+          s1 = Acc::add(s1, cw[t], v1[t]);
+        }
+      }
+      s0 = group_sum(s0, G);
+      s1 = group_sum(s1, G);
+      if (p == 0) {
+        float d0, d1;
+        if constexpr (sizeof(T) == 4) {
+          d0 = s0;
+          d1 = s1;
+        } else {
+          d0 = (float)(cnorm + s0);
+          d1 = (float)(cnorm + s1);
+        }
+        if (i0 < C0) {
+          cand_id[i0] = id0 >= 0 ? (uint32_t)id0 : ~0u;
+          cand_d[i0] = id0 >= 0 ? __float_as_uint(d0) : ~0u;
+        }
+        if (i1 < C0) {
+          cand_id[i1] = id1 >= 0 ? (uint32_t)id1 : ~0u;
+          cand_d[i1] = id1 >= 0 ? __float_as_uint(d1) : ~0u;
+        }
+      }
+    }
+    // (the rank loop reads the table four keys at a time)
+    if (tid < 4 && C0 + tid < kMaxCand && C0 + tid < ((C0 + 3) & ~3)) cand_id[C0 + tid] = cand_d[C0 + tid] = ~0u;
+    for (int i = tid; i < C0; i += kPruneThreads) sorted[i] = kPadKey;
+    __syncthreads();
+    for (int i = tid; i < C0; i += kPruneThreads) {
+      const uint64_t key = ((uint64_t)cand_d[i] << 32) | cand_id[i];
+      int rank = 0;
+      for (int k = 0; k < C0; k += 4) {
+        const uint4 kd = *reinterpret_cast<const uint4*>(cand_d + k);
+        const uint4 ki = *reinterpret_cast<const uint4*>(cand_id + k);
+        rank += (((uint64_t)kd.x << 32) | ki.x) < key ? 1 : 0;
+        rank += (((uint64_t)kd.y << 32) | ki.y) < key ? 1 : 0;
+        rank += (((uint64_t)kd.z << 32) | ki.z) < key ? 1 : 0;
+        rank += (((uint64_t)kd.w << 32) | ki.w) < key ? 1 : 0;
+      }
+      if (key != kPadKey) sorted[rank] = key;
+    }
+    __syncthreads();
+    // compact: places 0..255 by the four waves, then 256..511
+    uint64_t kept[2];
+    uint64_t in[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const int i = s * kPruneThreads + tid;
+      in[s] = i < C0 ? sorted[i] : kPadKey;
+      kept[s] = __ballot(in[s] != kPadKey);
+      if (lane == 0) counts[s * kWaves + wave] = (int)__popcll(kept[s]);
+    }
+    __syncthreads();
+    int C = 0;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      for (int w = 0; w < kWaves; w++) {
+        if (w == wave && in[s] != kPadKey) {
+          const int pos = C + (int)__popcll(kept[s] & ((1ull << lane) - 1));
+          if (pos < a.cmax) keys[pos] = in[s];
+        }
+        C += counts[s * kWaves + w];
+      }
+    }
+    C = min(C, a.cmax);
+    __syncthreads();  // the table and the sorted keys are overwritten by the rows below
+
+    int out_n = 0;
+    if (C <= L.R) {
+      for (int i = tid; i < C; i += kPruneThreads) cnb[1 + i] = (uint32_t)keys[i];
+      out_n = C;
+    } else {
+      // stage the candidate rows (and their norms) in LDS, fetched as above
+      for (int r0 = wave * 2 * rpr; r0 < C; r0 += kWaves * 2 * rpr) {
+        const int i0 = r0 + sub, i1 = r0 + rpr + sub;
+        const int64_t id0 = i0 < C ? (int64_t)(uint32_t)keys[i0] : center;
+        const int64_t id1 = i1 < C ? (int64_t)(uint32_t)keys[i1] : center;
+        const uint32_t* x0 = reinterpret_cast<const uint32_t*>(node_rec(L, id0));
+        const uint32_t* x1 = reinterpret_cast<const uint32_t*>(node_rec(L, id1));
+        AccT n0 = 0, n1 = 0;
+        for (int k0 = 0; k0 < kk; k0 += 4) {
+          uint32_t v0[4], v1[4];
+#pragma unroll
+          for (int t = 0; t < 4; t++) {
+            const int w = p + G * (k0 + t);
+            const bool ok = k0 + t < kk && w < ds4;
+            v0[t] = ok ? x0[w] : 0u;
+            v1[t] = ok ? x1[w] : 0u;
+          }
+#pragma unroll
+          for (int t = 0; t < 4; t++) {
+            const int w = p + G * (k0 + t);
+            if (k0 + t < kk && w < w4) {
+              if (i0 < C) vecs[i0 * S + w] = v0[t];
+              if (i1 < C) vecs[i1 * S + w] = v1[t];
+            }
+            n0 = Acc::norm_add(n0, v0[t]);
+            n1 = Acc::norm_add(n1, v1[t]);
+          }
+        }
+        if constexpr (sizeof(T) != 4) {
+          n0 = group_sum(n0, G);
+          n1 = group_sum(n1, G);
+          if (p == 0) {
+            if (i0 < C) norms[i0] = n0;
+            if (i1 < C) norms[i1] = n1;
+          }
+        }
+      }
+      __syncthreads();
+      const int q4 = w4 / 4;
+      bool alive = tid < C;
+      const int j = alive ? tid : 0;
+      const float dpj = __uint_as_float((uint32_t)(keys[j] >> 32));
+      const int32_t nj = sizeof(T) == 4 ? 0 : norms[j];
+      uint4 row[KR > 0 ? KR : 1];
+      if constexpr (KR > 0) {
+#pragma unroll
+        for (int q = 0; q < KR; q++)
+          if (q < q4) row[q] = reinterpret_cast<const uint4*>(vecs + j * S)[q];
+      }
+      int i = 0;  // the first candidate is always taken
+      for (int buf = 0;; buf ^= 1) {
+        if (tid == 0) outl[out_n] = (uint32_t)keys[i];
+        out_n++;
+        if (out_n == L.R) break;
+        alive = alive && tid > i;
+        if (alive) {
+          const float dij =
+              row_dist<T, KR>(vecs + i * S, row, vecs + j * S, q4, sizeof(T) == 4 ? 0 : norms[i], nj);
+          if (a.alpha * dij <= dpj) alive = false;
+        }
+        const uint64_t m = __ballot(alive);
+        if (lane == 0) masks[buf * kWaves + wave] = m;
+        __syncthreads();
+        i = -1;
+#pragma unroll
+        for (int w = kWaves - 1; w >= 0; w--) {
+          const uint64_t mw = masks[buf * kWaves + w];
+          if (mw) i = w * kWave + __ffsll((long long)mw) - 1;
+        }
+        if (i < 0) break;
+      }
+      __syncthreads();
+      for (int t = tid; t < out_n; t += kPruneThreads) cnb[1 + t] = outl[t];
+    }
+    if (tid == 0) {
+      cnb[0] = (uint32_t)out_n;
+      a.pcnt[center] = 0;
+    }
+    __syncthreads();
   }
 }
 
@@ -1126,10 +1107,12 @@ qv_index* build_gpu_t(const T* d_base, int dtype, int64_t n, int dim, const qv_b
                                   (size_t)(max_batch * prm.R), 0, 64, st));
   HIP_OK(hipMalloc(&d_tmp.p, tmp_bytes));
 
-  // Prune wave geometry: rows of `stride` dwords (16-byte pieces, an odd
-  // number of them, so 16 lanes reading 16 different rows hit distinct banks),
-  // G lanes per cooperative row fetch, and the largest candidate capacity
-  // that keeps 4 waves per CU (2 for long rows).
+  // Prune geometry: rows of `stride` dwords (16-byte pieces, an odd number of
+  // them, so 16 lanes reading 16 different rows hit distinct banks), G lanes
+  // per cooperative row fetch, and the candidate capacity: the largest with
+  // which four prunes (two of long rows) fit a CU.  The capacity cuts the
+  // candidates, so it is part of what graph a build gives: its rule counts the
+  // rows, keys and lists only.
   const int ds4 = (int)(lay.data_size / 4);
   int stride4 = (ds4 + 3) / 4;
   if (stride4 % 2 == 0) stride4++;
@@ -1138,19 +1121,30 @@ qv_index* build_gpu_t(const T* d_base, int dtype, int64_t n, int dim, const qv_b
   while (fetch_lanes < 64 && fetch_lanes * 4 < ds4) fetch_lanes *= 2;
   int lds_cu = 0;
   HIP_OK(hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, device));
-  auto waves_at = [&](int c) {
-    const int bytes = (prune_lds_plan(c, stride, prm.R).total + 1023) & ~1023;
+  auto prunes_at = [&](int c) {
+    const int bytes = (prune_lds_plan(c, stride, prm.R).rule + 1023) & ~1023;
     return lds_cu / bytes;
   };
   int cmax = 256;
-  while (cmax > 192 && waves_at(cmax) < 4) cmax -= 8;
-  if (waves_at(cmax) < 4) {
+  while (cmax > 192 && prunes_at(cmax) < 4) cmax -= 8;
+  if (prunes_at(cmax) < 4) {
     cmax = 256;
-    while (cmax > 64 && waves_at(cmax) < 2) cmax -= 8;
+    while (cmax > 64 && prunes_at(cmax) < 2) cmax -= 8;
   }
   const size_t prune_lds = (size_t)prune_lds_plan(cmax, stride, prm.R).total;
-  HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(prune_kernel<T>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)prune_lds));
+  // the candidate's row in registers where its 16-byte pieces fit
+  const int q4 = (ds4 + 3) / 4;
+  void (*prune)(PruneArgs) = q4 <= 8 ? prune_kernel<T, 8> : prune_kernel<T, 0>;
+  if constexpr (sizeof(T) == 4) {
+    if (q4 > 8 && q4 <= 32) prune = q4 <= 24 ? prune_kernel<T, 24> : prune_kernel<T, 32>;
+  }
+  HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(prune), hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)prune_lds));
+  auto launch_prune = [&](const PruneArgs& args) {
+    hipLaunchKernelGGL(prune, dim3((unsigned)std::min<int64_t>(args.num_centers, 65536)), dim3(kPruneThreads), prune_lds,
+                       st, args);
+    HIP_OK(hipGetLastError());
+  };
 
   const int passes = std::max(1, std::min(2, prm.passes));
   // QV_BUILD_PROGRESS=1: a progress line on stderr at most every 10 s (long builds)
@@ -1187,8 +1181,7 @@ qv_index* build_gpu_t(const T* d_base, int dtype, int64_t n, int dim, const qv_b
       pa.cmax = cmax;
       pa.stride = stride;
       pa.G = fetch_lanes;
-      hipLaunchKernelGGL(prune_kernel<T>, dim3((unsigned)std::min<int64_t>(nb, 65536)), dim3(64), prune_lds, st, pa);
-      HIP_OK(hipGetLastError());
+      launch_prune(pa);
 
       HIP_OK(hipMemsetAsync(d_cnt.p, 0, 64, st));
       const int64_t np = nb * prm.R;
@@ -1228,9 +1221,7 @@ qv_index* build_gpu_t(const T* d_base, int dtype, int64_t n, int dim, const qv_b
           ra.heads = d_heads.as<int32_t>();
           ra.marks = d_marks.as<int32_t>();
           ra.num_pairs = (int64_t)nvalid;
-          hipLaunchKernelGGL(prune_kernel<T>, dim3((unsigned)std::min<unsigned>(nmarks, 65536u)), dim3(64),
-                             prune_lds, st, ra);
-          HIP_OK(hipGetLastError());
+          launch_prune(ra);
           HIP_OK(hipStreamSynchronize(st));
         }
       }
@@ -1266,9 +1257,7 @@ qv_index* build_gpu_t(const T* d_base, int dtype, int64_t n, int dim, const qv_b
       fa.cmax = cmax;
       fa.stride = stride;
       fa.G = fetch_lanes;
-      hipLaunchKernelGGL(prune_kernel<T>, dim3((unsigned)std::min<unsigned>(nflush, 65536u)), dim3(64), prune_lds,
-                         st, fa);
-      HIP_OK(hipGetLastError());
+      launch_prune(fa);
       HIP_OK(hipStreamSynchronize(st));
     }
   }
