@@ -190,9 +190,10 @@ using KernelFn = void (*)(SearchArgs);
 constexpr int kXlQ = 32;
 
 // Waves (queries) one shared-pivot workgroup holds at most, by beam positions
-// per lane and neighbour slots per lane: 16 (128 registers per wave), or 8
-// (256) for beams of more than 7 positions per lane and for two slots.
-__host__ __device__ constexpr int sp_max_waves(int Q, int NPL) { return Q <= 7 && NPL == 1 ? 16 : 8; }
+// per lane and neighbour slots per lane: 16 (128 registers per wave), 12 (168)
+// for two slots, whose hop takes about 150 with the next node's two code rows
+// per lane, or 8 (256) for beams of more than 7 positions per lane.
+__host__ __device__ constexpr int sp_max_waves(int Q, int NPL) { return Q <= 7 ? (NPL == 1 ? 16 : 12) : 8; }
 
 // Whether the per-query-LUT search of these sizes runs on the team kernel: one
 // neighbour slot per lane, code rows in registers, and a beam whose wave needs
@@ -541,9 +542,10 @@ struct Query {
 
   // TL: the wave is in tail mode (kTail): the ADC reads its own LUT.
   template <int PF, bool TL = false>
-  __device__ __forceinline__ int32_t hop(int32_t v, Tk& tk, Rec& nr, CodeRow<MC>& cr, bool& have,
+  __device__ __forceinline__ int32_t hop(int32_t v, Tk& tk, Rec& nr, CodeRow<MC> (&crs)[NPL], bool& have,
                                          int32_t nxt = -1) {
-    if constexpr (NPL == 2) return hop2<PF == 1>(v, tk, nr);
+    if constexpr (NPL == 2) return hop2<PF>(v, tk, nr, crs, have, nxt);
+    CodeRow<MC>& cr = crs[0];
     const int lane = opaque_lane();
     const int deg = tk.deg;
     evals += deg;
@@ -740,33 +742,49 @@ struct Query {
   // neighbour whose entry A pushed out of the beam would have landed at or
   // beyond ef anyway, and no id repeats within one adjacency list.  The
   // guessed successor is the first unvisited entry before A (its record is
-  // requested at the start), compared by key after B.
-  template <bool PF>
-  __device__ __forceinline__ int32_t hop2(int32_t v, Tk& tk, Rec& nr) {
+  // requested at the start), compared by key after B.  PF, have and nxt as in
+  // hop, without the neighbour code table (R <= 64 only): the next node's 128
+  // code rows are requested from its record's ids once the ADC is done with
+  // crs, and stay in flight through both merges.  (Waiting for the record and
+  // then the rows in every hop, 5,000 queries at ef = 64 and pipe width 2 over
+  // 300,000 x 128 uint8, R = 128, took 1.47 ms; 1.42 ms so, and 1.18 ms with
+  // the 12 waves per CU of sp_max_waves instead of 8.)
+  template <int PF>
+  __device__ __forceinline__ int32_t hop2(int32_t v, Tk& tk, Rec& nr, CodeRow<MC> (&crs)[NPL], bool& have,
+                                          int32_t nxt) {
     const int lane = opaque_lane();
     const int deg = tk.deg;
     evals += deg;
     const bool has0 = lane < deg, has1 = lane + kWave < deg;
     const uint32_t nbr0 = tk.nbr[0], nbr1 = tk.nbr[1];
     const uint8_t* rec = kD == 0 && a.dim > 32 * kVecPre ? record(v) : nullptr;
-    const bool spec = PF && u < sz;
+    const bool spec = PF == 1 && u < sz;
     const uint64_t spec_key = bu;
     float d0, d1;
-    if constexpr (MC > 0 && MC % 16 == 0) {
-      CodeRow<MC> c0, c1;
-      adc_load<MC>(c0, a.codes, nbr0);
-      adc_load<MC>(c1, a.codes, nbr1);
-      if constexpr (PF) fetch(spec ? (int32_t)key_id(bu) : v, lane, nr);
+    if constexpr (kRows) {
+      if (!(PF != 0 && have)) {
+        adc_load<MC>(crs[0], a.codes, nbr0);
+        adc_load<MC>(crs[1], a.codes, nbr1);
+      }
+      // (issued on every hop, as in hop)
+      if constexpr (PF == 1) fetch(spec ? (int32_t)key_id(bu) : v, lane, nr);
+      if constexpr (PF == 2) fetch(nxt >= 0 ? nxt : v, lane, nr);
       exact_and_topk(v, tk.part, rec, lane);
       if constexpr (SC > 0) {
-        d0 = adc_recompute<MC, SC, kQd>(c0, qd);
-        d1 = adc_recompute<MC, SC, kQd>(c1, qd);
+        d0 = adc_recompute<MC, SC, kQd>(crs[0], qd);
+        d1 = adc_recompute<MC, SC, kQd>(crs[1], qd);
       } else {
-        d0 = adc_sum_at0<MC>(c0);
-        d1 = adc_sum_at0<MC>(c1);
+        d0 = adc_sum_at0<MC>(crs[0]);
+        d1 = adc_sum_at0<MC>(crs[1]);
+      }
+      if constexpr (PF != 0) {
+        const int ndeg = read_lane_i32(nr.deg, 0);
+        adc_load<MC>(crs[0], a.codes, lane < ndeg ? nr.nbr[0] : 0u);
+        adc_load<MC>(crs[1], a.codes, lane + kWave < ndeg ? nr.nbr[1] : 0u);
       }
     } else {
-      if (PF && spec) fetch((int32_t)key_id(bu), lane, nr);
+      if (PF == 1 && spec) fetch((int32_t)key_id(bu), lane, nr);
+      if (PF == 2 && nxt >= 0) fetch(nxt, lane, nr);
       d0 = adc_row<MC>(a.codes + (int64_t)nbr0 * a.num_chunks, lut, a.num_chunks);
       d1 = adc_row<MC>(a.codes + (int64_t)nbr1 * a.num_chunks, lut, a.num_chunks);
       exact_and_topk(v, tk.part, rec, lane);
@@ -775,8 +793,10 @@ struct Query {
     const uint64_t k1 = has1 ? make_key(d1, nbr1, false) : sentinel_key(lane + kWave);
     bool hit = false;
     merge_select<false, false>(k0, has0, lane, nr, false, spec_key, hit);
-    const int32_t nx = merge_select<true, PF>(k1, has1, lane, nr, spec, spec_key, hit);
-    if constexpr (PF) take(nr, tk, lane);
+    const int32_t nx = merge_select<true, PF == 1>(k1, has1, lane, nr, spec, spec_key, hit);
+    if constexpr (PF == 1 && kRows) have = hit;
+    if constexpr (PF == 2 && kRows) have = nxt >= 0;
+    if constexpr (PF != 0) take(nr, tk, lane);
     return nx;
   }
 
@@ -1481,7 +1501,7 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
 
     NodeRec<T, NPL> nr;
     Taken<NPL> tk;
-    CodeRow<MC> cr;
+    CodeRow<MC> cr[NPL];
     bool have = false;
     // Tail mode probe (kTail): from every 32nd hop on, the wave requests its
     // workgroup's count of ended waves and reads it at its next probe, so the
@@ -1528,7 +1548,7 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
         have = false;
       }
       const int32_t nx = Qy.template hop<2, decltype(tl)::value>(v, tk, nr, cr, have, nxt);
-      pf = NPL == 1 ? nxt : -1;
+      pf = nxt;
       return nx;
     };
 
@@ -1703,9 +1723,9 @@ __global__ __launch_bounds__(kTeamWaves * 64) void search_kernel_team(SearchArgs
 // once and every wave recomputes the LUT entries it needs (chunks of SC
 // dimensions), so the CU's LDS serves more queries than with a 32 KB LUT per
 // query.  Beams of more than 7 positions per lane (ef > 448; their LDS beams
-// allow 3 to 7 queries per CU) and two neighbour slots per lane (two code
-// rows per lane in flight) take 8 waves at most, which leaves each wave up to
-// 256 registers.
+// allow 3 to 7 queries per CU) take 8 waves at most, which leaves each wave up
+// to 256 registers, and two neighbour slots per lane (two code rows per lane in
+// flight) 12 waves.
 template <class T, int Q, int MC, int SC, int NPL>
 __global__ __launch_bounds__(kWave * sp_max_waves(Q, NPL)) void search_kernel_sp(SearchArgs a) {
   extern __shared__ __align__(16) char smem[];
