@@ -987,7 +987,7 @@ void search(qv_index* ix, const float* queries, int64_t nq, int dim, int topk, i
   const int spc = lp.slots_per_cu;
   if (spc <= 0) fail(QV_EUNSUPPORTED, "search kernel does not fit on a compute unit");
   // Query slots (search.cu:393-399): num_blocks x queries_per_block.  Each slot
-  // is a one-wave workgroup, so the reference's Q-interleave -- a block
+  // is one wave (or its team), so the reference's Q-interleave -- a block
   // switching between its slots while one waits on memory -- is the CU's own
   // wave interleaving here.  Slots beyond what the device holds resident would
   // only wait for a free CU, and slots beyond the number of queries would find
