@@ -1069,9 +1069,11 @@ qv_index* build_gpu_t(const T* d_base, int dtype, int64_t n, int dim, const qv_b
                      st, G, d_base);
   HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(st));
-  std::unique_ptr<qv_index, void (*)(qv_index*)> ix(
-      make_index(device, lay, pq, pages.as<uint8_t>(), codes.as<uint8_t>(), false), release_index);
-  pages.p = codes.p = nullptr;  // the index's now
+  // (both buffers are make_index's from its first line on, also when it throws)
+  uint8_t *const d_pages = pages.as<uint8_t>(), *const d_codes = codes.as<uint8_t>();
+  pages.p = codes.p = nullptr;
+  std::unique_ptr<qv_index, void (*)(qv_index*)> ix(make_index(device, lay, pq, d_pages, d_codes, false),
+                                                     release_index);
 
   // insertion order: seeded Fisher-Yates
   std::vector<int32_t> order((size_t)n);
