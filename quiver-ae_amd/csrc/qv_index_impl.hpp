@@ -57,6 +57,7 @@ struct qv_index {
   // pinned, coherent: a host-buffer call's results as the kernel writes them,
   // ids [cap_q][cap_k] int32, dists [cap_q][cap_k] float, found [cap_q] int32
   void* h_results = nullptr;
+  int32_t team_waves = 0;  // tests only: waves the team kernel is launched with (0: its own number)
   std::vector<int32_t> last_hops;
   std::vector<double> last_lat_ms;  // per-query latency of the last search, query order
   // host copies of the PQ tables (for saving the index)
@@ -100,3 +101,9 @@ void search_record(qv_index* ix, const float* d_queries, int64_t nq, int ef,
                    const SearchRecord& rec, int32_t* d_hops, int num_blocks);
 
 }  // namespace qv
+
+extern "C" {
+// Sets the handle's team_waves.  Not part of the public ABI: the tests reach
+// the team kernel's check of its workgroup through it.
+void qv_index_set_team_waves(qv_index* ix, int32_t waves);
+}

@@ -787,6 +787,7 @@ LaunchPlan launch_plan(qv_index* ix, int ef, int want, int64_t need, int topk) {
   lut.team = team_kernel(P, M, npl) ? kTeamWaves : 1;
   lut.lds = lds_plan(M, d, P, true, ef, topk, lut.team > 1).total;
   lut.slots_per_cu = occupancy(ix->device, ix->lds_cu, lut.kern, lut.team, lut.lds);
+  if (lut.team > 1 && ix->team_waves > 0) lut.team = ix->team_waves;
   if (want == QV_KERNEL_LUT) return lut;
   const bool forced = want == QV_KERNEL_SHARED_PIVOTS;
   if (wide) {
@@ -872,6 +873,12 @@ static SearchArgs base_args(qv_index* ix) {
   return a;
 }
 
+// Fails on the error bits a launch left in counters[2].
+static void check_errors(int32_t bits) {
+  if (bits & kErrSpinTimeout) fail(QV_ETIMEDOUT, "search kernel watchdog: feed wait exceeded its limit");
+  if (bits & kErrWorkgroup) fail(QV_EHIP, "search kernel: launched without a query's evaluator waves");
+}
+
 // Whole-batch search over device queries that records every expanded node and
 // its exact distance (the greedy-search step of graph construction).
 void search_record(qv_index* ix, const float* d_queries, int64_t nq, int ef, const SearchRecord& rec,
@@ -919,6 +926,7 @@ void search_record(qv_index* ix, const float* d_queries, int64_t nq, int ef, con
   HIP_OK(hipStreamSynchronize(ix->stream));
   int32_t counters[4] = {0, 0, 0, 0};
   HIP_OK(hipMemcpy(counters, ix->d_counters, sizeof(counters), hipMemcpyDeviceToHost));
+  check_errors(counters[2]);
   if (counters[1] != nq)
     fail(QV_EHIP, "record search finished " + std::to_string(counters[1]) + " of " + std::to_string(nq) + " queries");
 }
@@ -1296,7 +1304,7 @@ void search(qv_index* ix, const float* queries, int64_t nq, int dim, int topk, i
   int32_t* const st_evals = st_stopped + ix->cap_q;
   int32_t counters[5];
   std::memcpy(counters, st_counters, sizeof(counters));
-  if (counters[2] & kErrSpinTimeout) fail(QV_ETIMEDOUT, "search kernel watchdog: feed wait exceeded its limit");
+  check_errors(counters[2]);
   if (timed_out || counters[1] < nq) {
     char buf[96];
     std::snprintf(buf, sizeof(buf), "quiver_search exceeded the %g second timeout", o.timeout_s);
@@ -1478,6 +1486,7 @@ void search_noalloc(qv_index* ix, const float* d_queries, int64_t nq, int dim, i
   unsigned long long tot[3] = {0, 0, 0};
   HIP_OK(hipMemcpy(c, counters, sizeof(c), hipMemcpyDeviceToHost));
   HIP_OK(hipMemcpy(tot, totals, sizeof(tot), hipMemcpyDeviceToHost));
+  check_errors(c[2]);
   if (c[1] != nq)
     fail(QV_EHIP, "search kernel finished " + std::to_string(c[1]) + " of " + std::to_string(nq) + " queries");
   if (rep) {
@@ -1503,6 +1512,8 @@ void search_noalloc(qv_index* ix, const float* d_queries, int64_t nq, int dim, i
 // ================================================================ C ABI ====
 
 extern "C" {
+
+void qv_index_set_team_waves(qv_index* ix, int32_t waves) { ix->team_waves = waves; }
 
 void qv_search_opts_default(qv_search_opts* o) {
   if (!o) return;

@@ -89,7 +89,7 @@ struct SearchArgs {
   int32_t* wg_done;
 };
 
-enum : int32_t { kErrSpinTimeout = 1 };
+enum : int32_t { kErrSpinTimeout = 1, kErrWorkgroup = 2 };
 
 // Device copies of the host's feed word: one 8-byte word per line, the lines
 // 4352 bytes apart so that the waiting waves' reads spread over many memory
@@ -676,19 +676,15 @@ struct Query {
     const uint64_t want = at == 0 ? tm.word[0] : tm.word[1];
     const char* const slot = tm.slot + at * kTeamSlot;
     uint64_t nkey, info;
-    // (bounded: an evaluator answers every request; the limit only keeps a
-    // broken launch from spinning, and fails the search)
-    for (uint32_t n = 0;; n++) {
+    // (ends: an evaluator waits for nothing but requests, and answers the last
+    // one; that the workgroup has its evaluators is checked when it starts)
+    while (true) {
       const uint64_t d = read_lane_u64(lds_get(tm.done + at), 0);
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       nkey = reinterpret_cast<const uint64_t*>(slot)[lane];
       info = *reinterpret_cast<const uint64_t*>(slot + kWave * 8);
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       if (d == want) break;
-      if (n > (1u << 22)) {
-        if (lane == 0) atomicOr(&a.counters[2], kErrSpinTimeout);
-        break;
-      }
     }
     const int deg = read_lane_i32((int)(uint32_t)info, 0);
     evals += deg;
@@ -1716,6 +1712,10 @@ __global__ __launch_bounds__(64) void search_kernel(SearchArgs a) {
 template <class T, int Q, int MC, bool WK = false>
 __global__ __launch_bounds__(kTeamWaves * 64) void search_kernel_team(SearchArgs a) {
   extern __shared__ __align__(16) char smem[];
+  if (blockDim.x != kTeamWaves * kWave) {  // no query is begun without the waves that answer for it
+    if (threadIdx.x == 0) atomicOr(&a.counters[2], kErrWorkgroup);
+    return;
+  }
   run_queries<T, Q, MC, 0, 1, WK, true>(a, smem, nullptr);
 }
 

@@ -6,6 +6,8 @@ not, both code row lengths, chunks of uneven width, every pipe-lane regime
 than the device holds at once."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -57,3 +59,42 @@ def test_team_kernel(indexes, dtype, dim, M, R, pipe, nq, ef, k, policy):
                     early_exit=O.EXIT_GPRUNING if policy == "gpruning" else O.EXIT_NONE)
     np.testing.assert_array_equal(ids, want[0])
     np.testing.assert_array_equal(dists, want[1])
+
+
+@pytest.mark.parametrize("pipe, nq, k, policy", [(1, 1, 10, "none"), (2, 300, 10, "gpruning"), (5, 40, 100, "none")])
+def test_launch_without_evaluators(indexes, pipe, nq, k, policy):
+    """A workgroup that lacks its evaluators begins no query (nothing would answer for it): the search fails with that
+    cause whichever way its queries are admitted, and nothing is left behind."""
+    import quiver
+    from quiver import _lib
+
+    print(f"[gpu] team kernel launched with one wave, pipe={pipe} nq={nq} k={k}", flush=True)
+    d, host, q = indexes("uint8", 128, 32, 64)
+    q = np.ascontiguousarray(q[:nq], np.float32)
+    index = quiver.IndexQuiver(d, data_type="uint8", pipe_width=pipe, search_kernel="lut")
+    L = _lib.load()
+    L.qv_index_set_team_waves.argtypes, L.qv_index_set_team_waves.restype = [C.c_void_p, C.c_int32], None
+    handle = index._library().handle()
+    dq, out = _lib.DeviceBuffer(q.nbytes).upload(q), [_lib.DeviceBuffer(nq * k * 4) for _ in range(2)]
+    o = _lib.default_search_opts()
+    o.pipe_width, o.kernel, o.device_buffers = pipe, _lib.QV_KERNEL_LUT, 1
+
+    def on_device(entry):
+        return entry(handle, dq.ptr, nq, q.shape[1], k, 128, C.byref(o), out[0].ptr, out[1].ptr, None, None)
+
+    L.qv_index_set_team_waves(handle, 1)
+    with pytest.raises(_lib.QuiverError, match="without a query's evaluator waves"):
+        index.search(q, topk=k, ef_search=128, early_exit_policy=policy)
+    for admission in (_lib.QV_ADMIT_STREAMING, _lib.QV_ADMIT_BATCH, _lib.QV_ADMIT_STATIC):
+        o.admission = admission
+        assert on_device(L.qv_search) == _lib.QV_EHIP
+    assert on_device(L.qv_search_noalloc) == _lib.QV_EHIP
+    L.qv_index_set_team_waves(handle, 0)
+    ids, dists = index.search(q, topk=k, ef_search=128, early_exit_policy=policy)
+    index.close()
+    want = O.search(host, q, k, 128, pipe_width=pipe,
+                    early_exit=O.EXIT_GPRUNING if policy == "gpruning" else O.EXIT_NONE)
+    np.testing.assert_array_equal(ids, want[0])
+    np.testing.assert_array_equal(dists, want[1])
+    for b in (dq, *out):
+        b.close()
