@@ -7,6 +7,7 @@
 #include "qv_common.hpp"
 #include "qv_device.hpp"
 #include "qv_hip_util.hpp"
+#include "qv_index_impl.hpp"
 
 using namespace qv;
 using namespace qv::dev;
@@ -42,10 +43,12 @@ __device__ __forceinline__ void gt_offer(uint64_t& tk, int k, uint64_t key) {
 
 // Block (query group, base slice): 4 waves stream the slice, each lane one base
 // row at a time, distances to kGtQ queries in fp32 (exact for 8-bit data).
+// which: (direct kernels) the call's numbers of the nq queries, null for all.
 template <class T>
 __global__ __launch_bounds__(256) void gt_kernel(const T* __restrict__ base, int64_t n, int dim,
-                                                 const float* __restrict__ queries, int64_t nq, int k,
-                                                 int64_t slice, int S, uint64_t* __restrict__ part) {
+                                                 const float* __restrict__ queries, const int64_t* __restrict__ which,
+                                                 int64_t nq, int k, int64_t slice, int S,
+                                                 uint64_t* __restrict__ part) {
   extern __shared__ __align__(16) char smem[];
   float* q = reinterpret_cast<float*>(smem);
   uint64_t* xk = reinterpret_cast<uint64_t*>(q + kGtQ * dim);
@@ -54,7 +57,7 @@ __global__ __launch_bounds__(256) void gt_kernel(const T* __restrict__ base, int
   const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   for (int i = tid; i < kGtQ * dim; i += 256) {
     const int64_t qi = q0 + i / dim;
-    q[i] = qi < nq ? queries[qi * dim + (i % dim)] : 0.f;
+    q[i] = qi < nq ? queries[(which ? which[qi] : qi) * dim + (i % dim)] : 0.f;
   }
   __syncthreads();
   uint64_t tk[kGtQ];
@@ -109,15 +112,16 @@ __global__ __launch_bounds__(256) void gt_kernel(const T* __restrict__ base, int
   }
 }
 
-__global__ void gt_final_kernel(const uint64_t* __restrict__ part, int64_t nq, int S, int k,
-                                int32_t* __restrict__ ids, float* __restrict__ dists) {
+__global__ void gt_final_kernel(const uint64_t* __restrict__ part, const int64_t* __restrict__ which, int64_t nq, int S,
+                                int k, int32_t* __restrict__ ids, float* __restrict__ dists) {
   const int lane = lane_id();
   for (int64_t qi = blockIdx.x; qi < nq; qi += gridDim.x) {
     uint64_t tk = kPadKey;
     for (int s = 0; s < S; s++) gt_offer(tk, k, lane < k ? part[(qi * S + s) * k + lane] : kPadKey);
     if (lane < k) {
-      ids[qi * k + lane] = tk == kPadKey ? -1 : (int32_t)(uint32_t)tk;
-      dists[qi * k + lane] = tk == kPadKey ? __int_as_float(0x7f800000) : __uint_as_float((uint32_t)(tk >> 32));
+      const int64_t at = (which ? which[qi] : qi) * k + lane;
+      ids[at] = tk == kPadKey ? -1 : (int32_t)(uint32_t)tk;
+      dists[at] = tk == kPadKey ? __int_as_float(0x7f800000) : __uint_as_float((uint32_t)(tk >> 32));
     }
   }
 }
@@ -145,7 +149,8 @@ __device__ __forceinline__ uint32_t dot4(uint32_t a, uint32_t b, uint32_t acc) {
 
 template <class T>
 __global__ __launch_bounds__(256) void gt_int_kernel(const T* __restrict__ base, int64_t n, int dim,
-                                                     const float* __restrict__ queries, int64_t nq, int k,
+                                                     const float* __restrict__ queries,
+                                                     const int64_t* __restrict__ which, int64_t nq, int k,
                                                      int64_t slice, int S, uint64_t* __restrict__ part) {
   __shared__ __align__(16) uint32_t rows[kGtTile * kGtStride];
   __shared__ int32_t norms[kGtTile];
@@ -153,6 +158,7 @@ __global__ __launch_bounds__(256) void gt_int_kernel(const T* __restrict__ base,
   const int64_t qi = (int64_t)blockIdx.x * 256 + tid;
   const int s = blockIdx.y;
   const int d4 = dim / 4;
+  const int64_t query = qi < nq && which ? which[qi] : qi;
   uint32_t qw[kGtWords];
 #pragma unroll
   for (int w = 0; w < kGtWords; w++) {
@@ -160,7 +166,7 @@ __global__ __launch_bounds__(256) void gt_int_kernel(const T* __restrict__ base,
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const int j = 4 * w + e;
-      const int v = qi < nq && j < dim ? (int)queries[qi * dim + j] : 0;
+      const int v = qi < nq && j < dim ? (int)queries[query * dim + j] : 0;
       packed |= ((uint32_t)v & 0xffu) << (8 * e);
     }
     qw[w] = packed;
@@ -275,8 +281,13 @@ __global__ void gt_query_check(const float* __restrict__ q, int64_t count, int32
 // (S = 4^m, a few hundred rows) and keeps them all; level j the rows whose
 // number modulo S lies in [w, 4 w), w = 4^(j - 1), so every level scans three
 // times the rows of all before it, spread over the whole base, and about 3 k
-// of them pass the k-th distance found so far.  A list that overflows all the
-// same (data ordered against the period) sends the call to the direct kernels.
+// of them pass the k-th distance found so far.
+// Queries the scan cannot finish (8-bit: no whole numbers of the element type;
+// a list that overflows: data ordered against the period, more than a list of
+// float rows within the bound's slack of the k-th) are left out of its further
+// levels and go to the direct kernels, by themselves, as soon as the next
+// level's list is known not to hold them (gt_pick_kernel); once half of a batch
+// has left, all of it does and its scans end early.
 //
 // What bounds it: the matrix pipes need 4 x 32 cycles per 32 x 32 pairs of 128
 // bytes (1.25 M of the last level's 3.1 M cycles at the sizes below), the rest
@@ -303,6 +314,23 @@ constexpr int kGtPool = 128;         // candidates a wave gathers in LDS before 
 constexpr float kGtEps = 1.0f / 4096.0f;
 constexpr float kGtHuge = 1e37f;     // |x|^2 above this: the row or query is never dropped
 constexpr int kGtDrop = -(1 << 29);  // (8-bit) accumulator start of rows past the end
+constexpr uint32_t kGtLeft = 1u << 31;  // count of a query that has left the scan (no list entry is written past cap)
+
+// A batch's queries that have left the scan.
+struct GtLeft {
+  int32_t count;  // of them
+  int32_t all;    // set with the count at `limit`: the whole batch leaves, its scans end early
+};
+// What the host reads at the end of a call.
+struct GtCall {
+  unsigned long long direct;  // queries listed for the direct kernels
+  int32_t fractional;         // set when an 8-bit index's query is no whole number of the element type
+  int32_t pad;
+};
+
+__device__ __forceinline__ void gt_leave(GtLeft* left, int limit) {
+  if (atomicAdd(&left->count, 1) + 1 >= limit) left->all = 1;
+}
 
 struct ScanArgs {
   const uint8_t* base;
@@ -319,7 +347,8 @@ struct ScanArgs {
   uint32_t* cnt;        // [padded nq] candidates listed
   uint64_t* list;       // [nq][cap] keys (8-bit) or row ids (float)
   int cap;
-  int32_t* over;        // set when a list overflows: the call is lost, its scans end early
+  GtLeft* left;
+  int limit;
 };
 
 // Base row of a level's row i: every S-th row at level 0, else row i of the
@@ -387,19 +416,21 @@ __device__ __forceinline__ gt_i4 gt_shift(gt_i4 v, int w0, int nwords) {
 }
 
 // Queries into the scan's operand layout, with their norms, an open threshold
-// and an empty list; *lost is set when an 8-bit index's query is not a whole
-// number of the element type's range (the direct kernel takes those).  One
-// wave per query slot; slots past nq never match.
+// and an empty list; an 8-bit index's query that is not a whole number of the
+// element type's range leaves the scan here.  One wave per query slot; slots
+// past nq never match.
 template <class T, int KS>
 __global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ queries, int64_t nq, int dim,
                                                      uint8_t* __restrict__ qp, uint32_t* __restrict__ qn,
                                                      uint32_t* __restrict__ thr, uint64_t* __restrict__ tkey,
-                                                     uint32_t* __restrict__ cnt, int32_t* __restrict__ lost) {
+                                                     uint32_t* __restrict__ cnt, GtLeft* __restrict__ left, int limit,
+                                                     GtCall* __restrict__ call) {
   using K = GtKind<T>;
   const int lane = lane_id();
   const int64_t q = blockIdx.x;
   const bool live = q < nq;
   uint8_t* const out = qp + q * (int64_t)(K::kPlanes * KS * 32);
+  bool fractional = false;
   if constexpr (K::kFloat) {
     float s = 0.f;
     if (lane < KS * 2) {
@@ -439,16 +470,20 @@ __global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ q
       s = __builtin_amdgcn_sdot4((int)packed, (int)packed, s, false);
       reinterpret_cast<uint32_t*>(out)[w] = packed;
     }
-    if (wrong) *lost = 1;
+    fractional = __ballot(wrong) != 0;
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
     if (lane == 0) {
       qn[q] = (uint32_t)s;
-      thr[q] = (uint32_t)(live ? INT32_MIN : INT32_MAX);
+      thr[q] = (uint32_t)(live && !fractional ? INT32_MIN : INT32_MAX);
     }
   }
   if (lane == 0) {
     tkey[q] = kPadKey;
-    cnt[q] = 0;
+    cnt[q] = fractional ? kGtLeft : 0u;
+    if (fractional) {
+      call->fractional = 1;
+      gt_leave(left, limit);
+    }
   }
 }
 
@@ -567,8 +602,8 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
   int pooled = 0;
   auto flush = [&]() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    // a lost call adds nothing more (its counters would only be fought over)
-    if (pooled > 0 && __hip_atomic_load(a.over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) pooled = 0;
+    // a batch that has left adds nothing more (its counters would only be fought over)
+    if (pooled > 0 && __hip_atomic_load(&a.left->all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) pooled = 0;
     for (int i = lane; i < pooled; i += kWave) {
       const uint32_t at = pool_at[i];
       const int lq = wave * 32 * QT + pool_q[i];
@@ -584,7 +619,7 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
       if (take) {
         const uint32_t pos = atomicAdd(a.cnt + q, 1u);
         if (pos < (uint32_t)a.cap) a.list[q * a.cap + pos] = entry;
-        else *a.over = 1;
+        else if (pos == (uint32_t)a.cap) gt_leave(a.left, a.limit);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -629,7 +664,7 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
   int buf = 0;
   while (true) {
     const int64_t tn = t + a.slices;
-    const int32_t lost = __hip_atomic_load(a.over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int32_t lost = __hip_atomic_load(&a.left->all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (tn < tiles) request(tn);
     uint64_t parity = 0;
     if constexpr (!K::kFloat) parity = __ballot(odds[buf * kGtRows + lane] != 0);
@@ -714,14 +749,17 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
 // The k nearest of each query's listed rows, one wave per query: float rows
 // get their distance here (the direct kernel's fp32 chain over the
 // dimensions).  Before the last level: the threshold for the next one, and a
-// list of just these; at the last: the results.
+// list of just these, or the query leaves the scan; at the last: the results,
+// or for a query that has left its number in the direct kernels' list.
 template <class T>
 __global__ __launch_bounds__(256) void gt_pick_kernel(const uint8_t* __restrict__ base, int64_t row_bytes, int dim,
                                                       const float* __restrict__ queries, int64_t nq, int k,
                                                       const uint32_t* __restrict__ qn, uint32_t* __restrict__ thr,
                                                       uint64_t* __restrict__ tkey, uint32_t* __restrict__ cnt,
-                                                      uint64_t* __restrict__ list, int cap, bool last,
-                                                      int32_t* __restrict__ ids, float* __restrict__ dists) {
+                                                      uint64_t* __restrict__ list, int cap, int level, bool last,
+                                                      int32_t* __restrict__ ids, float* __restrict__ dists,
+                                                      GtLeft* __restrict__ left, int limit, int64_t first_query,
+                                                      GtCall* __restrict__ call, int64_t* __restrict__ direct) {
   __shared__ float qs[4][128];
   const int lane = lane_id(), wave = threadIdx.x / kWave;
   const int64_t q = (int64_t)blockIdx.x * 4 + wave;
@@ -731,7 +769,25 @@ __global__ __launch_bounds__(256) void gt_pick_kernel(const uint8_t* __restrict_
     __syncthreads();
   }
   if (q >= nq) return;
-  const int m = (int)min(cnt[q], (uint32_t)cap);
+  const uint32_t listed = cnt[q];
+  const bool all_left = __hip_atomic_load(&left->all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  // (a query whose list ran over, or is about to in the next level, leaves)
+  auto leave = [&]() {
+    if (lane == 0) {
+      if (last) {
+        direct[atomicAdd(&call->direct, 1ull)] = first_query + q;
+      } else if (listed < kGtLeft) {
+        if (listed <= (uint32_t)cap) gt_leave(left, limit);  // (past cap: counted by the scan)
+        cnt[q] = kGtLeft;
+        thr[q] = kFloat ? 0x7f800000u : (uint32_t)INT32_MAX;
+      }
+    }
+  };
+  if (all_left || listed > (uint32_t)cap) {
+    leave();
+    return;
+  }
+  const int m = (int)listed;
   uint64_t tk = kPadKey;
   for (int i0 = 0; i0 < m; i0 += kWave) {
     uint64_t key = kPadKey;
@@ -755,6 +811,7 @@ __global__ __launch_bounds__(256) void gt_pick_kernel(const uint8_t* __restrict_
           s = __fmaf_rn(d, d, s);
         }
         key |= (uint64_t)__float_as_uint(s) << 32;
+        if (level > 0 && !last && m > cap / 4) list[q * cap + i0 + lane] = key;  // (read again below)
       }
     }
     // the first 64 sorted at once, the others offered one by one
@@ -771,6 +828,23 @@ __global__ __launch_bounds__(256) void gt_pick_kernel(const uint8_t* __restrict_
       dists[q * k + lane] = tk == kPadKey ? __int_as_float(0x7f800000) : __uint_as_float((uint32_t)(tk >> 32));
     }
     return;
+  }
+  if constexpr (kFloat) {
+    // The next level has three times the rows of all before it, and of these
+    // the ones that would pass the new threshold are in the list: the ones not
+    // further than the k-th and the bound's slack (about 2 eps |q|^2 for a row
+    // near the query).
+    if (level > 0 && m > cap / 4) {
+      const float kth = __uint_as_float(read_lane_u32((uint32_t)(tk >> 32), k - 1));
+      const float reach = kth + 2.f * kGtEps * __uint_as_float(qn[q]);
+      int near = 0;
+      for (int i = lane; i < m; i += kWave) near += __uint_as_float((uint32_t)(list[q * cap + i] >> 32)) <= reach ? 1 : 0;
+      for (int off = 32; off > 0; off >>= 1) near += __shfl_xor(near, off);
+      if (3 * near > cap) {
+        leave();
+        return;
+      }
+    }
   }
   // the k found so far open the next level's list
   const uint64_t have = __ballot(lane < k && tk != kPadKey);
@@ -800,7 +874,7 @@ int grid_of(int64_t work, int block) {
 // The scan of one batch of queries, all levels (see above).
 template <class T, int KS, int QT>
 void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
-               float* d_dists, int cap, int64_t resident, uint8_t* work, int32_t* d_lost, hipStream_t st) {
+               float* d_dists, int cap, int64_t resident, uint8_t* work, GtLeft* left, int64_t first_query, GtCall* call, int64_t* direct, hipStream_t st) {
   const int64_t groups = (nq + 128 * QT - 1) / (128 * QT), padded = groups * 128 * QT;
   uint64_t* const list = reinterpret_cast<uint64_t*>(work);
   uint64_t* const tkey = list + nq * cap;
@@ -808,8 +882,9 @@ void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq
   uint32_t* const thr = qn + padded;
   uint32_t* const cnt = thr + padded;
   uint8_t* const qp = reinterpret_cast<uint8_t*>(cnt + padded);
+  const int limit = (int)((nq + 1) / 2);
   hipLaunchKernelGGL((gt_pack_kernel<T, KS>), dim3((unsigned)padded), dim3(64), 0, st, d_q, nq, dim, qp, qn, thr, tkey,
-                     cnt, d_lost);
+                     cnt, left, limit, call);
   HIP_OK(hipGetLastError());
   ScanArgs a{};
   a.base = reinterpret_cast<const uint8_t*>(d_base);
@@ -823,7 +898,8 @@ void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq
   a.cnt = cnt;
   a.list = list;
   a.cap = cap;
-  a.over = d_lost;
+  a.left = left;
+  a.limit = limit;
   int levels = 1;  // S = 4^(levels - 1): level 0 keeps all of its rows, at least k where n allows
   a.period = 1;
   while (n / (4 * a.period) >= (k <= 16 ? 64 : 256)) {
@@ -842,45 +918,89 @@ void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq
                        (size_t)gt_scan_lds<T>(KS, QT), st, a);
     HIP_OK(hipGetLastError());
     hipLaunchKernelGGL(gt_pick_kernel<T>, dim3((unsigned)((nq + 3) / 4)), dim3(256), 0, st, a.base, a.row_bytes, dim,
-                       d_q, nq, k, qn, thr, tkey, cnt, list, cap, l == levels - 1, d_ids, d_dists);
+                       d_q, nq, k, qn, thr, tkey, cnt, list, cap, l, l == levels - 1, d_ids, d_dists, left, limit,
+                       first_query, call, direct);
     HIP_OK(hipGetLastError());
   }
 }
 
+// The direct kernels for the nq queries listed in which (null: the call's
+// first nq).  whole: every one of them is a whole number of T's range.
+template <class T>
+void gt_direct(const T* d_base, int64_t n, int dim, const float* d_q, const int64_t* which, int64_t nq, int k,
+               int32_t* d_ids, float* d_dists, bool whole, hipStream_t st) {
+  uint64_t* part = nullptr;
+  int S = 0;
+  if (sizeof(T) == 1 && whole && dim <= 4 * kGtWords && k <= kGtMaxK) {
+    if constexpr (sizeof(T) == 1) {
+      const int64_t groups = (nq + 255) / 256;
+      const int64_t tiles = (n + kGtTile - 1) / kGtTile;
+      S = (int)std::max<int64_t>(1, std::min<int64_t>({256, tiles, (2048 + groups - 1) / groups}));
+      const int64_t slice = (tiles + S - 1) / S * kGtTile;
+      HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&part), sizeof(uint64_t) * (size_t)(nq * S * k), st));
+      hipLaunchKernelGGL(gt_int_kernel<T>, dim3((unsigned)groups, (unsigned)S), dim3(256), 0, st, d_base, n, dim, d_q,
+                         which, nq, k, slice, S, part);
+    }
+  } else {
+    S = (int)std::max<int64_t>(1, std::min<int64_t>(64, 4096 / std::max<int64_t>(1, (nq + kGtQ - 1) / kGtQ)));
+    const int64_t slice = (n + S - 1) / S;
+    HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&part), sizeof(uint64_t) * (size_t)(nq * S * k), st));
+    const size_t lds = (size_t)kGtQ * dim * 4 + (size_t)kGtQ * 4 * kWave * 8;
+    hipLaunchKernelGGL(gt_kernel<T>, dim3((unsigned)((nq + kGtQ - 1) / kGtQ), (unsigned)S), dim3(256), lds, st, d_base,
+                       n, dim, d_q, which, nq, k, slice, S, part);
+  }
+  HIP_OK(hipGetLastError());
+  hipLaunchKernelGGL(gt_final_kernel, dim3((unsigned)std::min<int64_t>(nq, 65536)), dim3(64), 0, st, part, which, nq, S,
+                     k, d_ids, d_dists);
+  HIP_OK(hipGetLastError());
+  HIP_OK(hipFreeAsync(part, st));
+}
+
+// The whole call by the scan, then the direct kernels for the queries that
+// left it (*direct of them).
 template <class T, int KS, int QT>
-bool gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
-                  float* d_dists, int device, hipStream_t st) {
+void gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
+                  float* d_dists, int device, int64_t* direct, hipStream_t st) {
   const void* const fn = reinterpret_cast<const void*>(&gt_scan_kernel<T, KS, QT>);
   HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, gt_scan_lds<T>(KS, QT)));
   int per_cu = 0, cus = 0;
   HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, (size_t)gt_scan_lds<T>(KS, QT)));
   HIP_OK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   const int cap = k <= 16 ? 512 : 2048;  // level 0 keeps up to 256 (1024) rows, a later one about 3 k
-  const int64_t batch = std::min<int64_t>(nq, kGtBatch);
+  const int64_t batch = std::min<int64_t>(nq, kGtBatch), batches = (nq + batch - 1) / batch;
   const int64_t padded = (batch + 128 * QT - 1) / (128 * QT) * (128 * QT);
-  const size_t bytes = (size_t)batch * cap * 8 + (size_t)padded * (8 + 12 + GtKind<T>::kPlanes * KS * 32) + 8;
+  const size_t lists = (size_t)batch * cap * 8 + (size_t)padded * (8 + 12 + GtKind<T>::kPlanes * KS * 32);
+  const size_t state = sizeof(GtCall) + (size_t)batches * sizeof(GtLeft);
   uint8_t* work = nullptr;
-  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&work), bytes, st));
-  int32_t* const d_lost = reinterpret_cast<int32_t*>(work + bytes - 8);
-  HIP_OK(hipMemsetAsync(d_lost, 0, 8, st));
-  for (int64_t q = 0; q < nq; q += batch)
+  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&work), lists + state + (size_t)nq * 8, st));
+  GtCall* const call = reinterpret_cast<GtCall*>(work + lists);
+  GtLeft* const left = reinterpret_cast<GtLeft*>(call + 1);
+  int64_t* const listed = reinterpret_cast<int64_t*>(left + batches);
+  HIP_OK(hipMemsetAsync(call, 0, state, st));
+  for (int64_t q = 0, b = 0; q < nq; q += batch, b++)
     gt_levels<T, KS, QT>(d_base, n, dim, d_q + q * dim, std::min(batch, nq - q), k, d_ids + q * k, d_dists + q * k, cap,
-                         (int64_t)per_cu * cus, work, d_lost, st);
-  int32_t lost = 0;
-  HIP_OK(hipMemcpyAsync(&lost, d_lost, sizeof(lost), hipMemcpyDeviceToHost, st));
-  HIP_OK(hipFreeAsync(work, st));
+                         (int64_t)per_cu * cus, work, left + b, q, call, listed, st);
+  GtCall host{};
+  HIP_OK(hipMemcpyAsync(&host, call, sizeof(host), hipMemcpyDeviceToHost, st));
   HIP_OK(hipStreamSynchronize(st));
-  return lost == 0;
+  *direct = (int64_t)host.direct;
+  if (host.direct > 0) {
+    gt_direct<T>(d_base, n, dim, d_q, listed, (int64_t)host.direct, k, d_ids, d_dists, !host.fractional, st);
+    HIP_OK(hipStreamSynchronize(st));
+  }
+  HIP_OK(hipFreeAsync(work, st));
 }
 
-// The matrix-core path where it applies; false (results to be recomputed) for
-// rows longer than its tiles, 8-bit queries that are no whole numbers of the
-// element type, or an overflowed candidate list.
+// The matrix-core path where it applies; false for rows longer than its tiles.
 template <class T>
 bool gt_matrix(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
-               float* d_dists, int device, hipStream_t st) {
+               float* d_dists, int device, int64_t* direct, hipStream_t st) {
   const bool few = nq <= 256;  // one query tile per wave: a workgroup then holds 128 queries, not 256 or 512
-#define QV_GT(KS, QT) return gt_matrix_ks<T, KS, QT>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, st)
+#define QV_GT(KS, QT)                                                                                       \
+  do {                                                                                                      \
+    gt_matrix_ks<T, KS, QT>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, direct, st);                \
+    return true;                                                                                            \
+  } while (0)
   if constexpr (sizeof(T) == 4) {
     if (dim > 128) return false;
     if (few) {
@@ -907,53 +1027,27 @@ bool gt_matrix(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq
 #undef QV_GT
 }
 
+// direct: how many of the queries the direct kernels answered.
 template <class T>
 void ground_truth_t(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
-                    float* d_dists, int device, hipStream_t st) {
-  if (gt_matrix<T>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, st)) return;
+                    float* d_dists, int device, int64_t* direct, hipStream_t st) {
+  if (gt_matrix<T>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, direct, st)) return;
+  *direct = nq;
+  int32_t bad = 1;
   if constexpr (sizeof(T) == 1) {
-    if (dim <= 4 * kGtWords && dim % 4 == 0 && k <= kGtMaxK) {
+    if (dim <= 4 * kGtWords && k <= kGtMaxK) {
       int32_t* d_bad = nullptr;
       HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&d_bad), sizeof(int32_t), st));
       HIP_OK(hipMemsetAsync(d_bad, 0, sizeof(int32_t), st));
       hipLaunchKernelGGL(gt_query_check<T>, dim3((unsigned)grid_of(nq * dim, 256)), dim3(256), 0, st, d_q, nq * dim,
                          d_bad);
       HIP_OK(hipGetLastError());
-      int32_t bad = 0;
       HIP_OK(hipMemcpyAsync(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost, st));
       HIP_OK(hipStreamSynchronize(st));
       HIP_OK(hipFreeAsync(d_bad, st));
-      if (!bad) {
-        const int64_t groups = (nq + 255) / 256;
-        const int64_t tiles = (n + kGtTile - 1) / kGtTile;
-        const int S = (int)std::max<int64_t>(1, std::min<int64_t>({256, tiles, (2048 + groups - 1) / groups}));
-        const int64_t slice = (tiles + S - 1) / S * kGtTile;
-        uint64_t* part = nullptr;
-        HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&part), sizeof(uint64_t) * (size_t)(nq * S * k), st));
-        hipLaunchKernelGGL(gt_int_kernel<T>, dim3((unsigned)groups, (unsigned)S), dim3(256), 0, st, d_base, n, dim,
-                           d_q, nq, k, slice, S, part);
-        HIP_OK(hipGetLastError());
-        hipLaunchKernelGGL(gt_final_kernel, dim3((unsigned)std::min<int64_t>(nq, 65536)), dim3(64), 0, st, part, nq,
-                           S, k, d_ids, d_dists);
-        HIP_OK(hipGetLastError());
-        HIP_OK(hipFreeAsync(part, st));
-        HIP_OK(hipStreamSynchronize(st));
-        return;
-      }
     }
   }
-  const int S = (int)std::max<int64_t>(1, std::min<int64_t>(64, 4096 / std::max<int64_t>(1, (nq + kGtQ - 1) / kGtQ)));
-  const int64_t slice = (n + S - 1) / S;
-  uint64_t* part = nullptr;
-  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&part), sizeof(uint64_t) * (size_t)(nq * S * k), st));
-  const size_t lds = (size_t)kGtQ * dim * 4 + (size_t)kGtQ * 4 * kWave * 8;
-  hipLaunchKernelGGL(gt_kernel<T>, dim3((unsigned)((nq + kGtQ - 1) / kGtQ), (unsigned)S), dim3(256), lds, st,
-                     d_base, n, dim, d_q, nq, k, slice, S, part);
-  HIP_OK(hipGetLastError());
-  hipLaunchKernelGGL(gt_final_kernel, dim3((unsigned)std::min<int64_t>(nq, 65536)), dim3(64), 0, st, part, nq, S,
-                     k, d_ids, d_dists);
-  HIP_OK(hipGetLastError());
-  HIP_OK(hipFreeAsync(part, st));
+  gt_direct<T>(d_base, n, dim, d_q, nullptr, nq, k, d_ids, d_dists, !bad, st);
   HIP_OK(hipStreamSynchronize(st));
 }
 
@@ -961,8 +1055,8 @@ void ground_truth_t(const T* d_base, int64_t n, int dim, const float* d_q, int64
 
 extern "C" {
 
-int qv_ground_truth(const void* d_base, int32_t data_type, int64_t n, int32_t dim, const float* d_queries,
-                    int64_t nq, int32_t k, int32_t* d_ids, float* d_dists, int device) {
+int qv_ground_truth_counted(const void* d_base, int32_t data_type, int64_t n, int32_t dim, const float* d_queries,
+                            int64_t nq, int32_t k, int32_t* d_ids, float* d_dists, int device, int64_t* direct) {
   return qv::guard([&] {
     if (!d_base || !d_queries || !d_ids || !d_dists) qv::fail(QV_EINVAL, "null argument");
     if (k <= 0 || k > 64 || n <= 0 || n > INT32_MAX || nq <= 0 || dim <= 0) qv::fail(QV_EINVAL, "bad shape");
@@ -970,14 +1064,20 @@ int qv_ground_truth(const void* d_base, int32_t data_type, int64_t n, int32_t di
     HIP_OK(hipSetDevice(device));
     hipStream_t st;
     HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    if (data_type == QV_UINT8)
-      ground_truth_t<uint8_t>(static_cast<const uint8_t*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, device, st);
-    else if (data_type == QV_INT8)
-      ground_truth_t<int8_t>(static_cast<const int8_t*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, device, st);
-    else
-      ground_truth_t<float>(static_cast<const float*>(d_base), n, dim, d_queries, nq, k, d_ids, d_dists, device, st);
+    auto go = [&](auto* base) {
+      ground_truth_t(base, n, dim, d_queries, nq, k, d_ids, d_dists, device, direct, st);
+    };
+    if (data_type == QV_UINT8) go(static_cast<const uint8_t*>(d_base));
+    else if (data_type == QV_INT8) go(static_cast<const int8_t*>(d_base));
+    else go(static_cast<const float*>(d_base));
     HIP_OK(hipStreamDestroy(st));
   });
+}
+
+int qv_ground_truth(const void* d_base, int32_t data_type, int64_t n, int32_t dim, const float* d_queries,
+                    int64_t nq, int32_t k, int32_t* d_ids, float* d_dists, int device) {
+  int64_t direct = 0;
+  return qv_ground_truth_counted(d_base, data_type, n, dim, d_queries, nq, k, d_ids, d_dists, device, &direct);
 }
 
 }  // extern "C"

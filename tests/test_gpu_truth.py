@@ -9,6 +9,8 @@ returned distances ascend and match the float64 ones rank by rank within that.
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -123,3 +125,79 @@ def test_float_rows_out_of_scale(lib):
         else:  # squares near the smallest normal numbers: ranks only, absolutely
             d = ((b2.astype(np.float64)[None] - q2.astype(np.float64)[:, None]) ** 2).sum(2)
             np.testing.assert_allclose(dists, np.sort(d, axis=1)[:, :10], rtol=98 * 2.0 ** -24, atol=96 * 2.0 ** -149)
+
+
+def _counted(lib, base, q, k):
+    """ids, distances, and how many of the queries the direct kernels answered."""
+    fn = lib.load().qv_ground_truth_counted
+    fn.restype, fn.argtypes = C.c_int32, lib.load().qv_ground_truth.argtypes + [C.POINTER(C.c_int64)]
+    n, dim = base.shape
+    nq = q.shape[0]
+    code = {"uint8": lib.QV_UINT8, "int8": lib.QV_INT8, "float32": lib.QV_FLOAT}[base.dtype.name]
+    bufs = [lib.DeviceBuffer(x.nbytes).upload(x) for x in (base, q)] + [lib.DeviceBuffer(nq * k * 4) for _ in range(2)]
+    direct = C.c_int64(-1)
+    lib.check(fn(bufs[0].ptr, code, n, dim, bufs[1].ptr, nq, k, bufs[2].ptr, bufs[3].ptr, 0, C.byref(direct)))
+    out = bufs[2].download(np.int32, (nq, k)), bufs[3].download(np.float32, (nq, k)), direct.value
+    for b in bufs:
+        b.close()
+    return out
+
+
+# the shapes of test_edges within the tiles' row lengths, and the largest 8-bit rows
+@pytest.mark.parametrize("dtype", ["uint8", "int8", "float32"])
+@pytest.mark.parametrize("n, nq, dim, k", [
+    (1, 1, 4, 1), (31, 3, 4, 40), (63, 31, 32, 5), (64, 33, 36, 64), (65, 128, 64, 16), (256, 129, 68, 17),
+    (1025, 257, 96, 10), (4097, 513, 100, 10), (16385, 256, 128, 16), (20001, 40, 128, 64), (5000, 20, 256, 64),
+])
+def test_the_scan_answers(lib, dtype, n, nq, dim, k):
+    """Ordinary data: no query is left to the direct kernels."""
+    print(f"[gpu] truth by the scan {dtype} n={n} nq={nq} dim={dim} k={k}", flush=True)
+    if dtype == "float32":
+        dim = min(dim, 128)
+    base, q = _rows(dtype, n, dim, n), _rows(dtype, nq, dim, n + 1).astype(np.float32)
+    ids, dists, direct = _counted(lib, base, q, k)
+    assert direct == 0
+    _check(base, q, k, ids, dists)
+
+
+@pytest.mark.parametrize("what, direct", [
+    ("one fractional query", 1), ("fractional queries", 70), ("against the period", 70), ("rows near one query", 1),
+    ("each row repeated", 70), ("long float rows", 70),
+])
+def test_queries_that_leave_the_scan(lib, what, direct):
+    """Only the queries the scan cannot finish go to the direct kernels."""
+    print(f"[gpu] truth, {what}", flush=True)
+    base, q = _rows("uint8", 20000, 16, 3, 250), _rows("uint8", 70, 16, 4, 250).astype(np.float32)
+    if what == "one fractional query":
+        q[33, 5] += 0.25
+    elif what == "fractional queries":
+        q += 0.5
+    elif what == "against the period":  # 250 rows a sample takes are far, the 750 scanned next near
+        base = base[:16000]
+        base[::4] = 255
+    else:
+        base, q = _rows("float32", 20000, 132 if what == "long float rows" else 96, 5), _rows("float32", 70, 96, 6)
+        rng = np.random.default_rng(8)
+        if what == "rows near one query":  # as near as one another, more than a list holds
+            q = np.ascontiguousarray(base[::250][:70] + rng.standard_normal((70, 96)) / 2, np.float32)
+            base[rng.permutation(20000)[:3000]] = q[12] + 0.125
+        elif what == "each row repeated":
+            base = np.ascontiguousarray(np.repeat(base[:10], 2000, axis=0)[rng.permutation(20000)])
+        elif what == "long float rows":
+            q = _rows("float32", 70, 132, 6)
+    ids, dists, got = _counted(lib, base, q, 10)
+    assert got == direct
+    _check(base, q, 10, ids, dists)
+
+
+@pytest.mark.parametrize("dtype", ["uint8", "float32"])
+def test_query_batches(lib, dtype):
+    """More queries than one scan takes (32,768): the second batch has its own lists, results and queries that leave."""
+    nq = 32768 + 37
+    print(f"[gpu] truth {dtype} nq={nq}", flush=True)
+    base, q = _rows(dtype, 300, 4, 1), _rows(dtype, nq, 4, 2).astype(np.float32)
+    if dtype == "uint8":
+        q[[7, 32770], 1] += 0.5
+    ids, dists, direct = _counted(lib, base, q, 3)
+    assert direct == (2 if dtype == "uint8" else 0)
+    _check(base, q, 3, ids, dists)
