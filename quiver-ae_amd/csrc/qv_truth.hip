@@ -288,6 +288,10 @@ __global__ void gt_query_check(const float* __restrict__ q, int64_t count, int32
 // levels and go to the direct kernels, by themselves, as soon as the next
 // level's list is known not to hold them (gt_pick_kernel); once half of a batch
 // has left, all of it does and its scans end early.
+// The slack is relative to the norms, so float rows and queries are taken
+// relative to a point amid the data (gt_start_kernel); a distance does not
+// change.  (Per dimension the median of 16 rows: a few rows far out do not
+// move it, as they would a mean.)
 //
 // What bounds it: the matrix pipes need 4 x 32 cycles per 32 x 32 pairs of 128
 // bytes (1.25 M of the last level's 3.1 M cycles at the sizes below), the rest
@@ -314,6 +318,7 @@ constexpr int kGtPool = 128;         // candidates a wave gathers in LDS before 
 constexpr float kGtEps = 1.0f / 4096.0f;
 constexpr float kGtHuge = 1e37f;     // |x|^2 above this: the row or query is never dropped
 constexpr int kGtDrop = -(1 << 29);  // (8-bit) accumulator start of rows past the end
+constexpr int kGtCenter = 128;       // (float) dimensions of the point amid the data, zero past the rows'
 constexpr uint32_t kGtLeft = 1u << 31;  // count of a query that has left the scan (no list entry is written past cap)
 
 // A batch's queries that have left the scan.
@@ -347,6 +352,7 @@ struct ScanArgs {
   uint32_t* cnt;        // [padded nq] candidates listed
   uint64_t* list;       // [nq][cap] keys (8-bit) or row ids (float)
   int cap;
+  const float* center;  // (float) [kGtCenter] point the rows and queries are taken relative to
   GtLeft* left;
   int limit;
 };
@@ -375,9 +381,12 @@ template <class T>
 constexpr int gt_row_lds(int KS) {
   return GtKind<T>::kPlanes * KS * 32 + 16;
 }
+// Lanes that stage one row, a 16-byte LDS piece of each plane per lane.
+constexpr int gt_lanes(int KS) { return KS <= 2 ? 4 : (KS <= 4 ? 8 : 16); }
 template <class T>
 constexpr int gt_scan_lds(int KS, int QT) {
-  return 2 * kGtRows * (gt_row_lds<T>(KS) + 8) + 4 * kGtPool * 12 + (GtKind<T>::kFloat ? 0 : 128 * QT * 12) + 8;
+  return 2 * kGtRows * (gt_row_lds<T>(KS) + 8) + 4 * kGtPool * 12 +
+         (GtKind<T>::kFloat ? gt_lanes(KS) * 32 : 128 * QT * 12) + 8;
 }
 
 // bf16 parts of 8 floats: hi rounded to nearest, lo the rounded rest.
@@ -415,6 +424,36 @@ __device__ __forceinline__ gt_i4 gt_shift(gt_i4 v, int w0, int nwords) {
   return v;
 }
 
+// Start of a call: its counts cleared (words of 4 bytes), and float: the point
+// amid the data, per dimension the median of 16 rows spread over the base (0
+// where there is none that is finite and not enormous).  One workgroup, a
+// thread per dimension.
+template <class T>
+__global__ __launch_bounds__(kGtCenter) void gt_start_kernel(const T* __restrict__ base, int64_t n, int dim,
+                                                             uint32_t* __restrict__ state, int64_t words,
+                                                             float* __restrict__ center) {
+  const int j = threadIdx.x;
+  for (int64_t i = j; i < words; i += kGtCenter) state[i] = 0u;
+  if constexpr (sizeof(T) == 4) {
+    constexpr int kRows = 16;
+    float c = 0.f;
+    if (j < dim) {
+      float v[kRows];
+#pragma unroll
+      for (int i = 0; i < kRows; i++) v[i] = base[(i * n / kRows) * dim + j];
+#pragma unroll
+      for (int i = 0; i < kRows; i++) {
+        int below = 0;
+#pragma unroll
+        for (int o = 0; o < kRows; o++) below += v[o] < v[i] || (v[o] == v[i] && o < i) ? 1 : 0;
+        if (below == kRows / 2) c = v[i];
+      }
+      if (!(fabsf(c) <= 1e15f)) c = 0.f;
+    }
+    center[j] = c;
+  }
+}
+
 // Queries into the scan's operand layout, with their norms, an open threshold
 // and an empty list; an 8-bit index's query that is not a whole number of the
 // element type's range leaves the scan here.  One wave per query slot; slots
@@ -423,8 +462,8 @@ template <class T, int KS>
 __global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ queries, int64_t nq, int dim,
                                                      uint8_t* __restrict__ qp, uint32_t* __restrict__ qn,
                                                      uint32_t* __restrict__ thr, uint64_t* __restrict__ tkey,
-                                                     uint32_t* __restrict__ cnt, GtLeft* __restrict__ left, int limit,
-                                                     GtCall* __restrict__ call) {
+                                                     uint32_t* __restrict__ cnt, const float* __restrict__ center,
+                                                     GtLeft* __restrict__ left, int limit, GtCall* __restrict__ call) {
   using K = GtKind<T>;
   const int lane = lane_id();
   const int64_t q = blockIdx.x;
@@ -438,7 +477,7 @@ __global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ q
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         const int i = lane * 8 + j;
-        x[j] = live && i < dim ? queries[q * dim + i] : 0.f;
+        x[j] = live && i < dim ? queries[q * dim + i] - center[i] : 0.f;
         s = __fmaf_rn(x[j], x[j], s);
       }
       gt_b8 hi, lo;
@@ -500,7 +539,7 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
   using One = typename K::One;
   constexpr int P = K::kPlanes;
   constexpr int kPieces = KS * 2;                                                // per plane and row
-  constexpr int kGroup = kPieces <= 4 ? 4 : (kPieces <= 8 ? 8 : 16);             // lanes per staged row
+  constexpr int kGroup = gt_lanes(KS);
   constexpr int kRounds = kGtRows * kGroup / 256;
   constexpr int kLoads = K::kPieceBytes / 16;
   constexpr int kStride = gt_row_lds<T>(KS);
@@ -513,7 +552,8 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
   uint32_t* const pool_at = reinterpret_cast<uint32_t*>(pools + (threadIdx.x / kWave) * 3 * kGtPool);
   int32_t* const pool_q = reinterpret_cast<int32_t*>(pool_at + kGtPool);
   int32_t* const pool_sum = pool_q + kGtPool;
-  // (8-bit) the workgroup's queries' key limits and norms
+  // (float) a.center; (8-bit) the workgroup's queries' key limits and norms
+  const float4* const center = reinterpret_cast<const float4*>(pools + 4 * 3 * kGtPool);
   uint64_t* const tkey = reinterpret_cast<uint64_t*>(pools + 4 * 3 * kGtPool);
   int32_t* const qnorm = reinterpret_cast<int32_t*>(tkey + 128 * QT);
   int32_t* const ended = reinterpret_cast<int32_t*>(smem + gt_scan_lds<T>(KS, QT) - 8);  // [2]
@@ -554,6 +594,8 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
     }
   };
   auto stage = [&](int64_t t, int buf) {
+    float4 c0, c1;
+    if constexpr (K::kFloat) c0 = center[2 * piece], c1 = center[2 * piece + 1];
 #pragma unroll
     for (int r = 0; r < kRounds; r++) {
       const int row = tid / kGroup + r * (256 / kGroup);
@@ -563,8 +605,11 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
       if constexpr (K::kFloat) {
         float x[8];
 #pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = __int_as_float(in[r][e / 4][e % 4]);
+        x[0] -= c0.x, x[1] -= c0.y, x[2] -= c0.z, x[3] -= c0.w;
+        x[4] -= c1.x, x[5] -= c1.y, x[6] -= c1.z, x[7] -= c1.w;
+#pragma unroll
         for (int e = 0; e < 8; e++) {
-          x[e] = __int_as_float(in[r][e / 4][e % 4]);
           s = __fmaf_rn(x[e], x[e], s);
         }
         for (int off = 1; off < kGroup; off <<= 1) s += __shfl_xor(s, off);
@@ -653,7 +698,10 @@ __global__ __launch_bounds__(256, 2) void gt_scan_kernel(ScanArgs a) {
   int64_t t = slice;
   if (t >= tiles) return;  // the whole workgroup
   request(t);
-  if constexpr (!K::kFloat) {
+  if constexpr (K::kFloat) {
+    if (tid < kGroup * 8) reinterpret_cast<float*>(pools + 4 * 3 * kGtPool)[tid] = a.center[tid];
+    __syncthreads();
+  } else {
     for (int i = tid; i < 128 * QT; i += 256) {
       tkey[i] = a.tkey[(int64_t)group * (128 * QT) + i];
       qnorm[i] = (int32_t)a.qn[(int64_t)group * (128 * QT) + i];
@@ -874,7 +922,8 @@ int grid_of(int64_t work, int block) {
 // The scan of one batch of queries, all levels (see above).
 template <class T, int KS, int QT>
 void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
-               float* d_dists, int cap, int64_t resident, uint8_t* work, GtLeft* left, int64_t first_query, GtCall* call, int64_t* direct, hipStream_t st) {
+               float* d_dists, int cap, int64_t resident, uint8_t* work, const float* center, GtLeft* left,
+               int64_t first_query, GtCall* call, int64_t* direct, hipStream_t st) {
   const int64_t groups = (nq + 128 * QT - 1) / (128 * QT), padded = groups * 128 * QT;
   uint64_t* const list = reinterpret_cast<uint64_t*>(work);
   uint64_t* const tkey = list + nq * cap;
@@ -884,7 +933,7 @@ void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq
   uint8_t* const qp = reinterpret_cast<uint8_t*>(cnt + padded);
   const int limit = (int)((nq + 1) / 2);
   hipLaunchKernelGGL((gt_pack_kernel<T, KS>), dim3((unsigned)padded), dim3(64), 0, st, d_q, nq, dim, qp, qn, thr, tkey,
-                     cnt, left, limit, call);
+                     cnt, center, left, limit, call);
   HIP_OK(hipGetLastError());
   ScanArgs a{};
   a.base = reinterpret_cast<const uint8_t*>(d_base);
@@ -898,6 +947,7 @@ void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq
   a.cnt = cnt;
   a.list = list;
   a.cap = cap;
+  a.center = center;
   a.left = left;
   a.limit = limit;
   int levels = 1;  // S = 4^(levels - 1): level 0 keeps all of its rows, at least k where n allows
@@ -972,14 +1022,17 @@ void gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t
   const size_t lists = (size_t)batch * cap * 8 + (size_t)padded * (8 + 12 + GtKind<T>::kPlanes * KS * 32);
   const size_t state = sizeof(GtCall) + (size_t)batches * sizeof(GtLeft);
   uint8_t* work = nullptr;
-  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&work), lists + state + (size_t)nq * 8, st));
+  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&work), lists + state + (size_t)nq * 8 + kGtCenter * 4, st));
   GtCall* const call = reinterpret_cast<GtCall*>(work + lists);
   GtLeft* const left = reinterpret_cast<GtLeft*>(call + 1);
   int64_t* const listed = reinterpret_cast<int64_t*>(left + batches);
-  HIP_OK(hipMemsetAsync(call, 0, state, st));
+  float* const center = reinterpret_cast<float*>(listed + nq);
+  hipLaunchKernelGGL(gt_start_kernel<T>, dim3(1), dim3(kGtCenter), 0, st, d_base, n, dim, reinterpret_cast<uint32_t*>(call),
+                     (int64_t)state / 4, center);
+  HIP_OK(hipGetLastError());
   for (int64_t q = 0, b = 0; q < nq; q += batch, b++)
     gt_levels<T, KS, QT>(d_base, n, dim, d_q + q * dim, std::min(batch, nq - q), k, d_ids + q * k, d_dists + q * k, cap,
-                         (int64_t)per_cu * cus, work, left + b, q, call, listed, st);
+                         (int64_t)per_cu * cus, work, center, left + b, q, call, listed, st);
   GtCall host{};
   HIP_OK(hipMemcpyAsync(&host, call, sizeof(host), hipMemcpyDeviceToHost, st));
   HIP_OK(hipStreamSynchronize(st));

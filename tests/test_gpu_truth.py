@@ -162,10 +162,10 @@ def test_the_scan_answers(lib, dtype, n, nq, dim, k):
 
 @pytest.mark.parametrize("what, direct", [
     ("one fractional query", 1), ("fractional queries", 70), ("against the period", 70), ("rows near one query", 1),
-    ("each row repeated", 70), ("long float rows", 70),
+    ("each row repeated", 70), ("common offset", 0), ("common offset, rows far out", 0), ("long float rows", 70),
 ])
 def test_queries_that_leave_the_scan(lib, what, direct):
-    """Only the queries the scan cannot finish go to the direct kernels."""
+    """Only the queries the scan cannot finish go to the direct kernels; a common offset is no reason to."""
     print(f"[gpu] truth, {what}", flush=True)
     base, q = _rows("uint8", 20000, 16, 3, 250), _rows("uint8", 70, 16, 4, 250).astype(np.float32)
     if what == "one fractional query":
@@ -185,6 +185,10 @@ def test_queries_that_leave_the_scan(lib, what, direct):
             base = np.ascontiguousarray(np.repeat(base[:10], 2000, axis=0)[rng.permutation(20000)])
         elif what == "long float rows":
             q = _rows("float32", 70, 132, 6)
+        else:
+            base, q = base + np.float32(300), q + np.float32(300)
+            if what == "common offset, rows far out":
+                base[::5000] = 1e12  # among the rows the scan's origin is taken from
     ids, dists, got = _counted(lib, base, q, 10)
     assert got == direct
     _check(base, q, 10, ids, dists)
