@@ -1007,9 +1007,10 @@ void gt_direct(const T* d_base, int64_t n, int dim, const float* d_q, const int6
 }
 
 // The whole call by the scan, then the direct kernels for the queries that
-// left it (*direct of them).
+// left it (*direct of them).  false: nothing was launched, its memory (lists of
+// 4 KB a query up to k = 16, of 16 KB beyond) could not be had.
 template <class T, int KS, int QT>
-void gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
+bool gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
                   float* d_dists, int device, int64_t* direct, hipStream_t st) {
   const void* const fn = reinterpret_cast<const void*>(&gt_scan_kernel<T, KS, QT>);
   HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, gt_scan_lds<T>(KS, QT)));
@@ -1022,7 +1023,13 @@ void gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t
   const size_t lists = (size_t)batch * cap * 8 + (size_t)padded * (8 + 12 + GtKind<T>::kPlanes * KS * 32);
   const size_t state = sizeof(GtCall) + (size_t)batches * sizeof(GtLeft);
   uint8_t* work = nullptr;
-  HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&work), lists + state + (size_t)nq * 8 + kGtCenter * 4, st));
+  const hipError_t got =
+      hipMallocAsync(reinterpret_cast<void**>(&work), lists + state + (size_t)nq * 8 + kGtCenter * 4, st);
+  if (got == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return false;
+  }
+  HIP_OK(got);
   GtCall* const call = reinterpret_cast<GtCall*>(work + lists);
   GtLeft* const left = reinterpret_cast<GtLeft*>(call + 1);
   int64_t* const listed = reinterpret_cast<int64_t*>(left + batches);
@@ -1042,18 +1049,16 @@ void gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t
     HIP_OK(hipStreamSynchronize(st));
   }
   HIP_OK(hipFreeAsync(work, st));
+  return true;
 }
 
-// The matrix-core path where it applies; false for rows longer than its tiles.
+// The matrix-core path where it applies; false for rows longer than its tiles
+// and where its memory cannot be had.
 template <class T>
 bool gt_matrix(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
                float* d_dists, int device, int64_t* direct, hipStream_t st) {
   const bool few = nq <= 256;  // one query tile per wave: a workgroup then holds 128 queries, not 256 or 512
-#define QV_GT(KS, QT)                                                                                       \
-  do {                                                                                                      \
-    gt_matrix_ks<T, KS, QT>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, direct, st);                \
-    return true;                                                                                            \
-  } while (0)
+#define QV_GT(KS, QT) return gt_matrix_ks<T, KS, QT>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, direct, st)
   if constexpr (sizeof(T) == 4) {
     if (dim > 128) return false;
     if (few) {

@@ -5,6 +5,8 @@
 //   alloc_failure_test build  a GPU build refused its i-th allocation, for
 //                             every i the call reaches, fails and frees
 //                             nothing twice
+//   alloc_failure_test truth  ground truth whose first allocation (the matrix
+//                             scan's lists) is refused still runs
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
@@ -119,8 +121,29 @@ static int build_refused() {
   return reached >= 20 ? 0 : 1;
 }
 
+static int truth_refused() {
+  const int64_t n = 5000, nq = 20;
+  const int32_t dim = 32, k = 50;
+  std::vector<float> base((size_t)n * dim, 1.f), q((size_t)nq * dim, 2.f), dists((size_t)nq * k);
+  std::vector<int32_t> ids((size_t)nq * k);
+  for (int32_t type : {QV_UINT8, QV_INT8, QV_FLOAT}) {
+    for (refuse = 0; refuse <= 1; refuse++) {
+      allocs = launches = 0;
+      const int rc = qv_ground_truth(base.data(), type, n, dim, q.data(), nq, k, ids.data(), dists.data(), 0);
+      if (rc != QV_OK || launches < 2 || !live.empty() || double_frees != 0) {
+        std::printf("type %d, allocation %ld refused: status %d (%s), %ld launches, %zu allocations left\n", type, refuse,
+                    rc, qv_last_error(), launches, live.size());
+        return 1;
+      }
+    }
+  }
+  std::printf("ground truth ran without its first allocation\n");
+  return 0;
+}
+
 int main(int argc, char** argv) {
   if (argc == 2 && std::strcmp(argv[1], "build") == 0) return build_refused();
-  std::fprintf(stderr, "usage: alloc_failure_test build\n");
+  if (argc == 2 && std::strcmp(argv[1], "truth") == 0) return truth_refused();
+  std::fprintf(stderr, "usage: alloc_failure_test build|truth\n");
   return 2;
 }
