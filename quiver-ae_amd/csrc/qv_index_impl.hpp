@@ -107,7 +107,9 @@ extern "C" {
 // the team kernel's check of its workgroup through it.
 void qv_index_set_team_waves(qv_index* ix, int32_t waves);
 // qv_ground_truth that also says how many of its queries the direct kernels
-// answered (as little part of the public ABI).
+// answered, and with scan_small takes the matrix scan however small the call
+// (as little part of the public ABI).
 int qv_ground_truth_counted(const void* d_base, int32_t data_type, int64_t n, int32_t dim, const float* d_queries,
-                            int64_t nq, int32_t k, int32_t* d_ids, float* d_dists, int device, int64_t* direct);
+                            int64_t nq, int32_t k, int32_t* d_ids, float* d_dists, int device, int32_t scan_small,
+                            int64_t* direct);
 }

@@ -1085,11 +1085,28 @@ bool gt_matrix(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq
 #undef QV_GT
 }
 
+// Whether a call is too small for the scan's levels, whose launches and lists
+// cost more than they save.  Float rows: up to half a million pairs (1,000 rows
+// x 100 queries x 96: 0.16 ms direct, 0.19 by the scan; 1,000 x 1,000: 0.33 and
+// 0.26) over few rows, which the direct kernel spreads over 64 workgroups per 8
+// queries (4,000 rows x 1 query: 0.20 and 0.18).  8-bit rows with more queries than one
+// small workgroup of the scan takes (with fewer the scan is the faster one at
+// any size): five million pairs of the integer kernel (60 x 1,000 x 128: 0.20
+// and 0.26; 300 x 10,000: 0.31 and 0.34; 2,000 x 10,000: 0.44 and 0.37), of the
+// fp32 kernel 600,000 (300 x 300, k = 50: 0.25 and 0.28; 1,000 x 1,000: 0.39
+// and 0.34).
+template <class T>
+bool gt_small(int64_t n, int dim, int64_t nq, int k) {
+  if (sizeof(T) == 4) return n <= 2048 && n * nq <= 500000;
+  return dim <= 4 * kGtWords && nq > 256 && n * nq <= (k <= kGtMaxK ? 5000000 : 600000);
+}
+
 // direct: how many of the queries the direct kernels answered.
 template <class T>
 void ground_truth_t(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq, int k, int32_t* d_ids,
-                    float* d_dists, int device, int64_t* direct, hipStream_t st) {
-  if (gt_matrix<T>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, direct, st)) return;
+                    float* d_dists, int device, bool scan_small, int64_t* direct, hipStream_t st) {
+  if ((scan_small || !gt_small<T>(n, dim, nq, k)) &&
+      gt_matrix<T>(d_base, n, dim, d_q, nq, k, d_ids, d_dists, device, direct, st)) return;
   *direct = nq;
   int32_t bad = 1;
   if constexpr (sizeof(T) == 1) {
@@ -1114,7 +1131,8 @@ void ground_truth_t(const T* d_base, int64_t n, int dim, const float* d_q, int64
 extern "C" {
 
 int qv_ground_truth_counted(const void* d_base, int32_t data_type, int64_t n, int32_t dim, const float* d_queries,
-                            int64_t nq, int32_t k, int32_t* d_ids, float* d_dists, int device, int64_t* direct) {
+                            int64_t nq, int32_t k, int32_t* d_ids, float* d_dists, int device, int32_t scan_small,
+                            int64_t* direct) {
   return qv::guard([&] {
     if (!d_base || !d_queries || !d_ids || !d_dists) qv::fail(QV_EINVAL, "null argument");
     if (k <= 0 || k > 64 || n <= 0 || n > INT32_MAX || nq <= 0 || dim <= 0) qv::fail(QV_EINVAL, "bad shape");
@@ -1123,7 +1141,7 @@ int qv_ground_truth_counted(const void* d_base, int32_t data_type, int64_t n, in
     hipStream_t st;
     HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     auto go = [&](auto* base) {
-      ground_truth_t(base, n, dim, d_queries, nq, k, d_ids, d_dists, device, direct, st);
+      ground_truth_t(base, n, dim, d_queries, nq, k, d_ids, d_dists, device, scan_small != 0, direct, st);
     };
     if (data_type == QV_UINT8) go(static_cast<const uint8_t*>(d_base));
     else if (data_type == QV_INT8) go(static_cast<const int8_t*>(d_base));
@@ -1135,7 +1153,7 @@ int qv_ground_truth_counted(const void* d_base, int32_t data_type, int64_t n, in
 int qv_ground_truth(const void* d_base, int32_t data_type, int64_t n, int32_t dim, const float* d_queries,
                     int64_t nq, int32_t k, int32_t* d_ids, float* d_dists, int device) {
   int64_t direct = 0;
-  return qv_ground_truth_counted(d_base, data_type, n, dim, d_queries, nq, k, d_ids, d_dists, device, &direct);
+  return qv_ground_truth_counted(d_base, data_type, n, dim, d_queries, nq, k, d_ids, d_dists, device, 0, &direct);
 }
 
 }  // extern "C"

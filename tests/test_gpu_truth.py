@@ -127,16 +127,17 @@ def test_float_rows_out_of_scale(lib):
             np.testing.assert_allclose(dists, np.sort(d, axis=1)[:, :10], rtol=98 * 2.0 ** -24, atol=96 * 2.0 ** -149)
 
 
-def _counted(lib, base, q, k):
-    """ids, distances, and how many of the queries the direct kernels answered."""
+def _counted(lib, base, q, k, scan_small=0):
+    """ids, distances, and how many of the queries the direct kernels answered (scan_small: the scan is taken however
+    small the call)."""
     fn = lib.load().qv_ground_truth_counted
-    fn.restype, fn.argtypes = C.c_int32, lib.load().qv_ground_truth.argtypes + [C.POINTER(C.c_int64)]
+    fn.restype, fn.argtypes = C.c_int32, lib.load().qv_ground_truth.argtypes + [C.c_int32, C.POINTER(C.c_int64)]
     n, dim = base.shape
     nq = q.shape[0]
     code = {"uint8": lib.QV_UINT8, "int8": lib.QV_INT8, "float32": lib.QV_FLOAT}[base.dtype.name]
     bufs = [lib.DeviceBuffer(x.nbytes).upload(x) for x in (base, q)] + [lib.DeviceBuffer(nq * k * 4) for _ in range(2)]
     direct = C.c_int64(-1)
-    lib.check(fn(bufs[0].ptr, code, n, dim, bufs[1].ptr, nq, k, bufs[2].ptr, bufs[3].ptr, 0, C.byref(direct)))
+    lib.check(fn(bufs[0].ptr, code, n, dim, bufs[1].ptr, nq, k, bufs[2].ptr, bufs[3].ptr, 0, scan_small, C.byref(direct)))
     out = bufs[2].download(np.int32, (nq, k)), bufs[3].download(np.float32, (nq, k)), direct.value
     for b in bufs:
         b.close()
@@ -150,13 +151,30 @@ def _counted(lib, base, q, k):
     (1025, 257, 96, 10), (4097, 513, 100, 10), (16385, 256, 128, 16), (20001, 40, 128, 64), (5000, 20, 256, 64),
 ])
 def test_the_scan_answers(lib, dtype, n, nq, dim, k):
-    """Ordinary data: no query is left to the direct kernels."""
+    """Ordinary data: no query is left to the direct kernels, and both ways give the same bits."""
     print(f"[gpu] truth by the scan {dtype} n={n} nq={nq} dim={dim} k={k}", flush=True)
     if dtype == "float32":
         dim = min(dim, 128)
     base, q = _rows(dtype, n, dim, n), _rows(dtype, nq, dim, n + 1).astype(np.float32)
-    ids, dists, direct = _counted(lib, base, q, k)
+    ids, dists, direct = _counted(lib, base, q, k, 1)
     assert direct == 0
+    _check(base, q, k, ids, dists)
+    for got, want in zip(_truth(lib, base, q, k), (ids, dists)):
+        np.testing.assert_array_equal(got, want)
+
+
+# both sides of the small-call lines: pairs, rows and queries
+@pytest.mark.parametrize("dtype, n, nq, dim, k, small", [
+    ("float32", 1000, 500, 32, 10, True), ("float32", 1000, 501, 32, 10, False), ("float32", 2048, 3, 32, 10, True),
+    ("float32", 2049, 3, 32, 10, False), ("uint8", 500, 256, 16, 10, False), ("uint8", 500, 257, 16, 10, True),
+    ("uint8", 5000, 1000, 16, 16, True), ("uint8", 5000, 1001, 16, 16, False), ("int8", 600, 1000, 16, 17, True),
+    ("int8", 600, 1001, 16, 17, False), ("int8", 100, 300, 132, 10, False),
+])
+def test_small_calls(lib, dtype, n, nq, dim, k, small):
+    print(f"[gpu] truth, small call {dtype} n={n} nq={nq} dim={dim} k={k}", flush=True)
+    base, q = _rows(dtype, n, dim, n), _rows(dtype, nq, dim, n + 1).astype(np.float32)
+    ids, dists, direct = _counted(lib, base, q, k)
+    assert direct == (nq if small else 0)
     _check(base, q, k, ids, dists)
 
 
