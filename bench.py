@@ -536,10 +536,12 @@ def open_loop_leg(_lib, L, h, qf, dim, nq, ref_ids, ef, policy, pname, pipe, cap
     fractions of the device-resident closed-loop rate, past it until the
     backlog of a rate above what the launch sustains lifts P99 over 10 ms
     (one launch has no per-batch drain, so it sustains more than the
-    closed loop's rate); reported per point: offered and
+    closed loop's rate); logged per point: offered and
     achieved QPS, P50/P99, the kernel `auto` took, and whether every answer
-    equals the closed-loop one.  Per batch size: the highest offered rate
-    whose P99 is at most 10 ms."""
+    equals the closed-loop one.  Returned: how many points, whether every
+    answer of all of them did, and per batch size the point of the highest
+    offered rate whose P99 is at most 10 ms (all of the points would make the
+    result line 6 KB longer)."""
     reps_q = 30
     n = nq * reps_q
     q10 = np.ascontiguousarray(np.tile(qf, (reps_q, 1)), np.float32)
@@ -549,7 +551,8 @@ def open_loop_leg(_lib, L, h, qf, dim, nq, ref_ids, ef, policy, pname, pipe, cap
     want = np.tile(ref_ids, (reps_q, 1))
     fracs = (0.1, 0.25, 0.5, 0.75, 1.0, 1.1, 1.2, 1.3, 1.35, 1.4, 1.45, 1.5, 1.6)
     out = {"ef_search": ef, "early_exit": pname, "pipe_width": pipe, "arrivals": n,
-           "closed_loop_qps": round(capacity, 1), "points": [], "max_offered_qps_p99_le_10ms": {}}
+           "closed_loop_qps": round(capacity, 1), "points": 0, "ids_identical_to_closed_loop": True,
+           "max_offered_qps_p99_le_10ms": {}}
     for b in batches:
         best = None
         for f in fracs:
@@ -570,7 +573,8 @@ def open_loop_leg(_lib, L, h, qf, dim, nq, ref_ids, ef, policy, pname, pipe, cap
                    "p50_ms": round(rep.lat_p50_ms, 3), "p99_ms": round(rep.lat_p99_ms, 3),
                    "kernel": "shared-pivots" if rep.kernel == _lib.QV_KERNEL_SHARED_PIVOTS else "lut",
                    "ids_identical_to_closed_loop": same}
-            out["points"].append(row)
+            out["points"] += 1
+            out["ids_identical_to_closed_loop"] = out["ids_identical_to_closed_loop"] and same
             log(f"open loop batch={b:4d} offered={rate:10.0f} achieved={rep.qps:10.0f} p50={rep.lat_p50_ms:.3f} "
                 f"p99={rep.lat_p99_ms:.3f} kernel={row['kernel']} same={same}")
             if rep.lat_p99_ms <= 10.0 and (best is None or rate > best["offered_qps"]):
@@ -661,12 +665,12 @@ def adc_leg(_lib, L, ncodes: int, log) -> dict:
     log(f"gather alone: {gms:.3f} ms, {evals / gms / 1e6:.1f} G rows/s; ADC at {gms / ms:.1%} of that rate")
     # the access-rate matrix: the same ids over tables of 32 MB to 32 GB, rows
     # of 32-256 bytes, both load types, 1-4 rows in flight, 8-32 waves per CU
-    matrix = access_matrix(_lib, L, codes, ncodes, M, ids, evals, log)
+    matrix, cells = access_matrix(_lib, L, codes, ncodes, M, ids, evals, log)
     # rows of 32, 64, 128 and 256 bytes from the whole table, as the ADC
     # kernel reads (nontemporal, one row in flight, 32 waves per CU): a rate
     # that does not fall with the width means the gather pays per row
     widths = {}
-    for c in matrix["cells"]:
+    for c in cells:
         if (c["table_bytes"] == min(32_000_000_000, ncodes * M) and c["nontemporal"] and c["rows_in_flight"] == 1
                 and c["waves_per_cu"] == 32):
             widths[c["row_bytes"]] = {"ms": c["ms"], "rows_per_s": c["rows_per_s"], "gb_per_s": c["gb_per_s"]}
@@ -705,13 +709,15 @@ def adc_leg(_lib, L, ncodes: int, log) -> dict:
             "physical_frac_of_stream_read": round(phys_gbs / stream_gbs, 4)}
 
 
-def access_matrix(_lib, L, codes, ncodes, M, ids, n, log) -> dict:
+def access_matrix(_lib, L, codes, ncodes, M, ids, n, log) -> tuple[dict, list]:
     """The random row gather's rate over its shape: tables of 32 MB, 3.2 GB and
     32 GB (prefixes of the code table), rows of 32-256 bytes, nontemporal or
     default loads, 1, 2 or 4 rows in flight per lane group and 8, 16 or 32
     waves per CU (the last two swept for 32-byte rows only).  The same n
     uniform ids each time (mapped onto the table's rows); rows/s per cell,
-    the median of two timed launches after one untimed."""
+    the median of two timed launches after one untimed.  Returns what the
+    result line holds (the number of cells and the best one: all of them would
+    make it 18 KB longer) and the cells, which the log lists."""
     fold = _lib.DeviceBuffer(4)
     cells = []
     for table in (32_000_000, 3_200_000_000, 32_000_000_000):
@@ -741,7 +747,7 @@ def access_matrix(_lib, L, codes, ncodes, M, ids, n, log) -> dict:
         log(f"  table={c['table_bytes'] / 1e9:7.3f} GB row={c['row_bytes']:3d} nt={int(c['nontemporal'])} "
             f"per={c['rows_in_flight']} waves={c['waves_per_cu']:2d}: {c['rows_per_s'] / 1e9:6.1f} G rows/s "
             f"{c['gb_per_s']:7.0f} GB/s")
-    return {"cells": cells, "best_32b": best}
+    return {"cells": len(cells), "best_32b": best}, cells
 
 
 def cpu_leg(_lib, L, h, info, qf, ef, policy, pname, pipe, gpu_ids_all, gpu_dists_all, nq,

@@ -54,3 +54,25 @@ def test_small_bench_line():
     assert r["queries_per_launch"] == 30000 and 0 < r["frac"] < 1
     assert abs(r["frac"] - r["achieved"] / r["peak"]) < 1e-3
     assert out["latency_mode"] and out["latency_mode"][0]["batch"] == 1
+
+
+@pytest.mark.gpu
+def test_the_whole_line_is_short():
+    """Every leg's figures in one line that a captured output's last 16 KB still hold: the access matrix's cells and
+    the open loop's points are in the log, the line has the best of them."""
+    from quiver import _lib
+
+    if _lib.device_count() == 0:
+        pytest.skip("no GPU")
+    print("[gpu] bench.py small workload, every GPU leg, 4M codes", flush=True)
+    rc, out, err = _run("--workload", "small-1M-u8", "--n", "200000", "--steps", "1", "--warmup", "1", "--repeat", "2",
+                        "--no-cpu", "--adc-codes", "4000000")
+    assert rc == 0, err[-2000:]
+    adc, loop = out["adc"], out["open_loop"]
+    assert adc["access_matrix"]["cells"] > 50 and adc["access_matrix"]["best_32b"]["row_bytes"] == 32
+    assert set(adc["random_row_widths"]) == {"32", "64", "128", "256"}
+    assert err.count("G rows/s") > adc["access_matrix"]["cells"]
+    assert loop["points"] == 39 and loop["ids_identical_to_closed_loop"] is True
+    assert set(loop["max_offered_qps_p99_le_10ms"]) == {"1", "16", "256"}
+    assert err.count("open loop batch=") == loop["points"]
+    assert out["latency_mode"] and len(json.dumps(out)) < 12000
