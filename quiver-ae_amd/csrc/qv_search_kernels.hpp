@@ -118,7 +118,8 @@ __host__ __device__ inline int max_int(int x, int y) { return x > y ? x : y; }
 
 struct LdsPlan {
   int lut_off, qc_off, qu_off, beam_off, count_off, wide_off, total;
-  int slot_off, ctrl_off;  // team kernel: the evaluators' answers, the request words
+  // team kernel: the evaluators' answers, the request and done words, the query's number
+  int slot_off, ctrl_off, qid_off;
 };
 
 // Team kernel: a query's workgroup is one wave that owns the beam and
@@ -127,10 +128,16 @@ struct LdsPlan {
 constexpr int kTeamEval = 2;
 constexpr int kTeamWaves = 1 + kTeamEval;
 // LDS of one evaluator's answer: 64 keys, then the degree and the node's
-// exact distance.  The answers overlay the query copies where no wave reads
-// those after the LUT is built (dim <= 32 kVecPre).
+// exact distance.  The answers overlay what no wave reads after the LUT is
+// built: the first query copy and the first 32 kVecPre elements of the second,
+// which the lanes then hold.  Beyond that many dimensions the request and done
+// words lie there too and the query's number lies where the beam will be, so
+// that a team takes no more LDS than one wave and as many queries fit a CU
+// (M = 48, 192 dimensions, ef = 200: 53,760 bytes, three; with 1,104 bytes of
+// the team's own they were two, and 8,000 queries at pipe width 1 took 5.9 ms,
+// float 7.2 ms, against one wave's 5.7 and 6.8).
 constexpr int kTeamSlot = kWave * 8 + 16;
-constexpr int kTeamCtrl = 48;  // [kTeamEval] request words, [kTeamEval] done words, the query id
+constexpr int kTeamCtrl = 2 * kTeamEval * 8;  // [kTeamEval] request words, [kTeamEval] done words
 
 // Top-k entries a wave holds in its registers: entry i in lane i.  The
 // per-query-LUT kernel keeps entries 64 .. k - 1 of a larger k in LDS after
@@ -159,18 +166,25 @@ __host__ __device__ inline LdsPlan lds_plan(int num_chunks, int dim, int Q, bool
   p.qu_off = p.qc_off + dpad * 4;
   const bool overlay = !lut && dim <= 32 * kVecPre;
   p.beam_off = overlay ? p.qc_off : (p.qu_off + dpad * 4 + 15) & ~15;
-  p.slot_off = p.ctrl_off = 0;
-  if (team) {
-    p.slot_off = dim <= 32 * kVecPre ? p.qc_off : p.beam_off;
-    p.beam_off = max_int(p.beam_off, p.slot_off + kTeamEval * kTeamSlot);
+  p.slot_off = p.qc_off;
+  p.ctrl_off = p.slot_off + kTeamEval * kTeamSlot;
+  const bool team_ctrl = team && dim <= 32 * kVecPre;  // (then the words have a place of their own)
+  if (team_ctrl) {
+    p.beam_off = max_int(p.beam_off, p.ctrl_off);
+  } else if (team) {
+    // (the second copy moves up where the first one is short)
+    p.qu_off = max_int(p.qu_off, p.ctrl_off + kTeamCtrl - 32 * kVecPre * 4);
+    p.beam_off = (p.qu_off + dpad * 4 + 15) & ~15;
   }
+  p.qid_off = p.beam_off;
   const int beam_bytes = beam_cap(ef, Q, lut) * 8;
   p.count_off = p.beam_off + beam_bytes;  // (rank_counts: no overlay)
   p.total = p.beam_off + (overlay && 2 * dpad * 4 > beam_bytes ? 2 * dpad * 4 : beam_bytes) +
             (rank_counts(lut, Q) ? beam_cap(ef, Q, lut) * 4 : 0);
-  if (team) {
+  if (team_ctrl) {
     p.ctrl_off = p.total;
-    p.total += kTeamCtrl;
+    p.qid_off = p.ctrl_off + kTeamCtrl;
+    p.total += kTeamCtrl + 16;
   }
   p.wide_off = p.total;
   if (lut) p.total += wide_topk(topk) * 8;
@@ -651,6 +665,17 @@ struct Query {
   }
   static __device__ __forceinline__ uint64_t lds_get(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+
+  // The request word between queries: the last one's quit.
+  static __device__ __forceinline__ uint64_t idle_word(uint32_t number) {
+    return ((uint64_t)number << 32) | (uint32_t)kTeamQuit;
+  }
+  static __device__ __forceinline__ void team_idle(const Team& tm) {
+    for (int e = 0; e < kTeamEval; e++) {
+      lds_put(tm.req + e, idle_word(tm.number));
+      lds_put(tm.done + e, 0);
+    }
   }
 
   // Asks evaluator e for v unless one of them has it.
@@ -1301,9 +1326,12 @@ __device__ __forceinline__ void query_sync() {
 
 // Team kernel, every wave of the workgroup: the query into LDS, this wave's
 // chunks of the LUT, this lane's query elements.  The answers' slots and the
-// beam may be written once the last barrier is passed.
+// beam may be written once the last barrier is passed.  Beyond 32 kVecPre
+// dimensions the request words lie in the query copies: the beam's wave sets
+// them anew once every wave has what it needs of those, and the evaluators look
+// at them after another barrier.
 template <class Qu>
-__device__ __forceinline__ void team_query(const SearchArgs& a, Qu& Qy, const float* q) {
+__device__ __forceinline__ void team_query(const SearchArgs& a, Qu& Qy, const typename Qu::Team& team, const float* q) {
   for (int i = (int)threadIdx.x; i < a.dim; i += kTeamWaves * kWave) {
     const float c = query_elem(q, i) - a.centroid[i];
     Qy.qc[i] = c;
@@ -1313,6 +1341,10 @@ __device__ __forceinline__ void team_query(const SearchArgs& a, Qu& Qy, const fl
   load_query_pre(Qy.qu, a.dim, lane_id(), Qy.quv);
   build_lut_lds(Qy.qc, a.pivots_t, a.chunk_off, a.num_chunks, Qy.lut, (int)(threadIdx.x / kWave), kTeamWaves);
   __syncthreads();
+  if (a.dim > 32 * kVecPre) {
+    if (threadIdx.x == 0) Qu::team_idle(team);
+    __syncthreads();
+  }
 }
 
 // The persistent query loop of one wave: smem is its LDS area, piv the
@@ -1329,18 +1361,18 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     team.req = reinterpret_cast<uint64_t*>(smem + pl.ctrl_off);
     team.done = team.req + kTeamEval;
     team.slot = smem + pl.slot_off;
-    team_qid = reinterpret_cast<int32_t*>(team.done + kTeamEval);
+    team_qid = reinterpret_cast<int32_t*>(smem + pl.qid_off);
     team.number = 0;
     const int wave = (int)(threadIdx.x / kWave);
-    if (threadIdx.x < 2 * kTeamEval) team.req[threadIdx.x] = 0;  // ordered by the first barrier below
+    if (threadIdx.x == 0) Qu::team_idle(team);  // ordered by the first barrier below
     if (wave > 0) {
-      uint64_t seen = 0;
+      uint64_t seen = Qu::idle_word(0);
       while (true) {
         __syncthreads();  // the query's number is out
         const int32_t qid = *team_qid;
         if (qid < 0) return;
         Qu Qy(a, smem, piv);
-        team_query(a, Qy, a.queries + (int64_t)qid * a.dim);
+        team_query(a, Qy, team, a.queries + (int64_t)qid * a.dim);
         Qy.answer(team.req + wave - 1, team.done + wave - 1, team.slot + (wave - 1) * kTeamSlot, seen);
       }
     }
@@ -1430,7 +1462,7 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     // ---- query into LDS: q - mu for the LUT, fl(fl(q - mu) + mu) for the exact
     // distance (pq_device.cuh:18-20, 33-35).
     if constexpr (TM) {
-      team_query(a, Qy, q);
+      team_query(a, Qy, team, q);
 #pragma unroll
       for (int w = 0; w < kTeamEval; w++) team.word[w] = (uint64_t)(uint32_t)Qu::kTeamQuit;
     } else {
@@ -1660,7 +1692,7 @@ __device__ __forceinline__ void run_queries(const SearchArgs& a, char* smem, con
     if constexpr (TM) {
       // the evaluators go to the next query's barrier
       team.number++;
-      if (lane < kTeamEval) Qu::lds_put(team.req + lane, ((uint64_t)team.number << 32) | (uint32_t)Qu::kTeamQuit);
+      if (lane < kTeamEval) Qu::lds_put(team.req + lane, Qu::idle_word(team.number));
     }
     // ---- finish (kernel_q1.cuh:662-704)
     if (sr) {

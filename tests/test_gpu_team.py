@@ -61,6 +61,28 @@ def test_team_kernel(indexes, dtype, dim, M, R, pipe, nq, ef, k, policy):
     np.testing.assert_array_equal(dists, want[1])
 
 
+@pytest.mark.parametrize("dtype, dim, M, ef, k, per_cu", [
+    ("uint8", 192, 48, 200, 10, 3), ("float", 192, 48, 256, 10, 3), ("uint8", 256, 32, 448, 10, 4),
+    ("uint8", 132, 48, 256, 10, 3), ("float", 640, 32, 200, 10, 4), ("float", 144, 48, 65, 1, 3),
+])
+def test_full_device(indexes, dtype, dim, M, ef, k, per_cu):
+    """More queries than the device holds: as many on a CU as with one wave per query, every one right."""
+    import quiver
+    from quiver import _lib
+
+    print(f"[gpu] full device {dtype} d={dim} M={M} ef={ef} k={k}", flush=True)
+    d, host, q = indexes(dtype, dim, M, 16)
+    cus = C.c_int32()
+    _lib.check(_lib.load().qv_device_info(0, C.create_string_buffer(64), 64, C.byref(cus), C.byref(C.c_int64())))
+    index = quiver.IndexQuiver(d, data_type=dtype, pipe_width=1, search_kernel="lut")
+    ids, dists = index.search(q, topk=k, ef_search=ef, early_exit_policy="none")
+    index.close()
+    assert index.last_report["num_blocks"] == min(per_cu * cus.value, len(q))
+    want = O.search(host, q.astype(np.float32), k, ef, early_exit=O.EXIT_NONE)
+    np.testing.assert_array_equal(ids, want[0])
+    np.testing.assert_array_equal(dists, want[1])
+
+
 @pytest.mark.parametrize("pipe, nq, k, policy", [(1, 1, 10, "none"), (2, 300, 10, "gpruning"), (5, 40, 100, "none")])
 def test_launch_without_evaluators(indexes, pipe, nq, k, policy):
     """A workgroup that lacks its evaluators begins no query (nothing would answer for it): the search fails with that
