@@ -209,6 +209,11 @@ int beam_chunks_sp(int ef) {
   return q <= 7 ? q : (q <= 10 ? 10 : 16);
 }
 
+// LDS is given to workgroups in pieces of this many bytes (128 to a CU).  Seen:
+// a top-k of 160 beside a 48-chunk LUT (53,760 bytes) runs three queries on a
+// CU, 161 (53,824) two.
+constexpr int kLdsGranule = 1280;
+
 // Neighbour slots per lane for an index of max degree R.
 int slots_per_lane(int64_t R) { return R <= kWave ? 1 : 2; }
 
@@ -787,6 +792,25 @@ LaunchPlan launch_plan(qv_index* ix, int ef, int want, int64_t need, int topk) {
   lut.team = team_kernel(P, M, npl) ? kTeamWaves : 1;
   lut.lds = lds_plan(M, d, P, true, ef, topk, lut.team > 1).total;
   lut.slots_per_cu = occupancy(ix->device, ix->lds_cu, lut.kern, lut.team, lut.lds);
+  const KernelFn alone = lut.team > 1 && wide && npl == 1 ? pick_kernel_wide_one_wave(ix->lay.data_type, P, M) : nullptr;
+  if (alone) {
+    // A large top-k beside the LUT can leave the team, whose answers take up to
+    // 336 bytes more (lds_plan, dim <= 128), two queries per CU where one wave
+    // per query fits three: then a full device is better off with those.
+    // 8,000 queries x 96 floats, M = 48, top-128 at ef = 256, pipe widths 1, 2
+    // and 4: 6.4, 6.7 and 6.8 ms, the team 7.6, 6.5 and 7.0.  (Three instead of
+    // four: uint8, M = 32, top-280 at ef = 300: 6.7, 6.8 and 6.5, the team 6.2,
+    // 6.5 and 6.5.)  The counts are the LDS's own, which is given out in
+    // kLdsGranule bytes: the runtime's leave that out and say three for both.
+    const int lds = lds_plan(M, d, P, true, ef, topk).total;
+    const auto fit = [&](int bytes) { return ix->lds_cu / ((bytes + kLdsGranule - 1) / kLdsGranule * kLdsGranule); };
+    if (2 * fit(lds) >= 3 * fit(lut.lds) && need > (int64_t)fit(lut.lds) * ix->num_cus) {
+      lut.kern = alone;
+      lut.team = 1;
+      lut.lds = lds;
+      lut.slots_per_cu = occupancy(ix->device, ix->lds_cu, alone, 1, lds);
+    }
+  }
   if (lut.team > 1 && ix->team_waves > 0) lut.team = ix->team_waves;
   if (want == QV_KERNEL_LUT) return lut;
   const bool forced = want == QV_KERNEL_SHARED_PIVOTS;

@@ -224,6 +224,9 @@ KernelFn pick_kernel_sp_deep(int dtype, int Q, int M);
 // Per-query-LUT kernels for a top-k above 64 (qv_search_wide.hip): Q = 2, 4,
 // 7, 10 or 16 (from wide_beam_chunks), one or two neighbour slots per lane.
 KernelFn pick_kernel_wide(int dtype, int Q, int M, int npl);
+// The one-wave kernel of a size that pick_kernel_wide gives the team kernel
+// for, one neighbour slot per lane; null where there is none.
+KernelFn pick_kernel_wide_one_wave(int dtype, int Q, int M);
 __host__ __device__ inline int wide_beam_chunks(int ef) {
   return ef <= 128 ? 2 : (ef <= 256 ? 4 : (ef <= 448 ? 7 : (ef <= 640 ? 10 : (ef <= 1024 ? 16 : kXlQ))));
 }

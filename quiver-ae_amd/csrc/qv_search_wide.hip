@@ -21,6 +21,14 @@ KernelFn wide_mc(int M) {
   return search_kernel<T, Q, 0, NPL, true>;
 }
 
+// The one-wave kernel where it holds half again as many queries per CU as the
+// team (launch_plan): 48-chunk LUTs beside beams of four positions per lane,
+// three instead of two.
+template <class T>
+KernelFn one_wave(int Q, int M) {
+  return Q == 4 && M == 48 ? search_kernel<T, 4, 48, 1, true> : nullptr;
+}
+
 template <class T, int NPL>
 KernelFn wide_q(int Q, int M) {
   switch (Q) {
@@ -47,6 +55,12 @@ KernelFn pick_kernel_wide(int dtype, int Q, int M, int npl) {
   if (dtype == QV_UINT8) return wide_npl<uint8_t>(Q, M, npl);
   if (dtype == QV_INT8) return wide_npl<int8_t>(Q, M, npl);
   return wide_npl<float>(Q, M, npl);
+}
+
+KernelFn pick_kernel_wide_one_wave(int dtype, int Q, int M) {
+  if (dtype == QV_UINT8) return one_wave<uint8_t>(Q, M);
+  if (dtype == QV_INT8) return one_wave<int8_t>(Q, M);
+  return one_wave<float>(Q, M);
 }
 
 }  // namespace sk

@@ -64,6 +64,10 @@ def test_team_kernel(indexes, dtype, dim, M, R, pipe, nq, ef, k, policy):
 @pytest.mark.parametrize("dtype, dim, M, ef, k, per_cu", [
     ("uint8", 192, 48, 200, 10, 3), ("float", 192, 48, 256, 10, 3), ("uint8", 256, 32, 448, 10, 4),
     ("uint8", 132, 48, 256, 10, 3), ("float", 640, 32, 200, 10, 4), ("float", 144, 48, 65, 1, 3),
+    # a large top-k: the team while it holds as many, one wave per query where that holds three for two, and the
+    # team again where both hold two (the runtime counts three)
+    ("float", 96, 48, 256, 112, 3), ("float", 96, 48, 256, 113, 3), ("uint8", 100, 48, 200, 150, 3),
+    ("float", 96, 48, 256, 160, 3), ("float", 96, 48, 256, 161, 3), ("uint8", 132, 48, 256, 113, 3),
 ])
 def test_full_device(indexes, dtype, dim, M, ef, k, per_cu):
     """More queries than the device holds: as many on a CU as with one wave per query, every one right."""
