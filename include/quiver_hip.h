@@ -75,7 +75,7 @@ typedef struct {
   int32_t data_type;      /* QV_UINT8 / QV_FLOAT / QV_INT8 */
   int32_t num_chunks;     /* PQ M */
   int32_t device;
-  int32_t slots_per_cu;   /* concurrent queries (waves) per CU of the kernel a full
+  int32_t slots_per_cu;   /* concurrent queries per CU of the kernel a full
                              batch takes at ef <= 64 */
   int64_t device_bytes;   /* HBM held by the index */
   int64_t nav_nodes;      /* nodes of the loaded nav graph (0: none, entry = medoid) */
@@ -188,8 +188,9 @@ void qv_index_close(qv_index* index);
 typedef struct {
   int32_t num_blocks;        /* --num-blocks; 0 fills the GPU */
   int32_t queries_per_block; /* --queries-per-block, 1..8: num_blocks x this many query
-                                slots (search.cu:393-399), one wave each; the launch
-                                stops at the device's resident capacity */
+                                slots (search.cu:393-399), one wave each or the three
+                                waves of one workgroup; the launch stops at the
+                                device's resident capacity */
   int32_t pipe_width;        /* --pipe-width, 1..16 */
   int32_t early_exit;        /* QV_EXIT_NONE / QV_EXIT_GPRUNING */
   int32_t gpruning_warmup;   /* 10 in the reference CLI */

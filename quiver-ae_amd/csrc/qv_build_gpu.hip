@@ -95,7 +95,7 @@ __global__ __launch_bounds__(64) void pq_mean_kernel(const T* __restrict__ base,
   if (j >= dim) return;
   if constexpr (sizeof(T) == 1) {
     const int64_t per = (ns + gridDim.y - 1) / gridDim.y, r0 = blockIdx.y * per, r1 = min(ns, r0 + per);
-    int s = 0;  // at most 2^18 rows of 8 bits
+    int s = 0;  // (under 2^23 rows of 8 bits)
 #pragma unroll 8
     for (int64_t i = r0; i < r1; i++) s += (int)base[(int64_t)rows[i] * dim + j];
     atomicAdd(reinterpret_cast<unsigned long long*>(sums + j), (unsigned long long)(long long)s);

@@ -205,8 +205,9 @@ constexpr int kXlQ = 32;
 
 // Waves (queries) one shared-pivot workgroup holds at most, by beam positions
 // per lane and neighbour slots per lane: 16 (128 registers per wave), 12 (168)
-// for two slots, whose hop takes about 150 with the next node's two code rows
-// per lane, or 8 (256) for beams of more than 7 positions per lane.
+// for two slots, whose hop takes 132 to 150 with the next node's two code rows
+// per lane (103 to 126 without them, hop2), or 8 (256) for beams of more than 7
+// positions per lane.
 __host__ __device__ constexpr int sp_max_waves(int Q, int NPL) { return Q <= 7 ? (NPL == 1 ? 16 : 12) : 8; }
 
 // Whether the per-query-LUT search of these sizes runs on the team kernel: one
@@ -649,8 +650,8 @@ struct Query {
   // the slot; a slot is asked again only after its last answer is not needed.
   //
   // Measured (1M x 128 uint8, ef = 208, pipe width 2): a hop 1.80 -> 1.45 us
-  // for one query, a call 414 -> 346 us; 16 queries of 96 floats in host
-  // buffers 340 -> 263 us; 3,000 top-100 queries over 1,024 teams 2.15 -> 1.72
+  // for one query, a call 414 -> 338 us; 16 queries of 96 floats in host
+  // buffers 333 -> 252 us; 3,000 top-100 queries over 1,024 teams 2.21 -> 1.69
   // ms.  What is left of the hop, in cycles: 440 for the answer, 350 for the
   // next request and the top-k, 950 for the ranks in the beam, 270 for the
   // selection, 980 for the merge.
@@ -772,7 +773,10 @@ struct Query {
   // crs, and stay in flight through both merges.  (Waiting for the record and
   // then the rows in every hop, 5,000 queries at ef = 64 and pipe width 2 over
   // 300,000 x 128 uint8, R = 128, took 1.47 ms; 1.42 ms so, and 1.18 ms with
-  // the 12 waves per CU of sp_max_waves instead of 8.)
+  // the 12 waves per CU of sp_max_waves instead of 8.  The two together at pipe
+  // widths 1, 2 and 4: ef = 64 1.41, 1.45, 1.50 -> 1.23, 1.18, 1.21 ms; ef = 256
+  // 3.76, 4.03, 4.06 -> 3.15, 3.00, 3.02; ef = 448 6.30, 6.77, 6.82 -> 6.29, 6.34,
+  // 6.47.  Not tried: 16 waves without the rows.)
   template <int PF>
   __device__ __forceinline__ int32_t hop2(int32_t v, Tk& tk, Rec& nr, CodeRow<MC> (&crs)[NPL], bool& have,
                                           int32_t nxt) {

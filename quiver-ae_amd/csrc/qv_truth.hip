@@ -274,7 +274,8 @@ __global__ void gt_query_check(const float* __restrict__ q, int64_t count, int32
 //     q.x, the norms' and the ranked distance's own rounding together are
 //     below kGtEps (|q|^2 + |x|^2) for dim <= 128 (2^-15 |q||x| of dropped
 //     parts and 2^-15.4 of 3 x 128 accumulations, twice, plus 2^-16 for the
-//     sums of squares: under 2^-12.9), so a row is only dropped when its
+//     sums of squares and 2^-22 for the differences to the point below: under
+//     2^-12.9), so a row is only dropped when its
 //     distance is above the threshold whatever the rounding.  The candidates'
 //     distances are the fp32 chain of the direct kernel.
 // Thresholds come from the rows already scanned.  Level 0 takes every S-th row
