@@ -284,7 +284,7 @@ __global__ void gt_query_check(const float* __restrict__ q, int64_t count, int32
 // times the rows of all before it, spread over the whole base, and about 3 k
 // of them pass the k-th distance found so far.
 // Queries the scan cannot finish (8-bit: no whole numbers of the element type;
-// a list that overflows: data ordered against the period, more than a list of
+// float: a norm that is no number or overflows; a list that overflows: data ordered against the period, more than a list of
 // float rows within the bound's slack of the k-th) are left out of its further
 // levels and go to the direct kernels, by themselves, as soon as the next
 // level's list is known not to hold them (gt_pick_kernel); once half of a batch
@@ -317,7 +317,7 @@ constexpr int kGtRows = 64;          // base rows per LDS tile
 constexpr int64_t kGtBatch = 32768;  // queries per scan: the lists' memory (4 KB a query up to k = 16, 16 KB beyond)
 constexpr int kGtPool = 128;         // candidates a wave gathers in LDS before it appends them to the lists
 constexpr float kGtEps = 1.0f / 4096.0f;
-constexpr float kGtHuge = 1e37f;     // |x|^2 above this: the row or query is never dropped
+constexpr float kGtHuge = 1e37f;     // |x|^2 above this: the row is never dropped, the query leaves the scan
 constexpr int kGtDrop = -(1 << 29);  // (8-bit) accumulator start of rows past the end
 constexpr int kGtCenter = 128;       // (float) dimensions of the point amid the data, zero past the rows'
 constexpr uint32_t kGtLeft = 1u << 31;  // count of a query that has left the scan (no list entry is written past cap)
@@ -456,9 +456,11 @@ __global__ __launch_bounds__(kGtCenter) void gt_start_kernel(const T* __restrict
 }
 
 // Queries into the scan's operand layout, with their norms, an open threshold
-// and an empty list; an 8-bit index's query that is not a whole number of the
-// element type's range leaves the scan here.  One wave per query slot; slots
-// past nq never match.
+// and an empty list.  An 8-bit index's query that is not a whole number of the
+// element type's range leaves the scan here, and a float one without a finite
+// norm that its bound could use: as zeros, since a NaN reaches any threshold
+// (one such query of 2,000 x 500,000 x 96 would take the scan from 1.0 to 6.1
+// ms).  One wave per query slot; slots past nq never match.
 template <class T, int KS>
 __global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ queries, int64_t nq, int dim,
                                                      uint8_t* __restrict__ qp, uint32_t* __restrict__ qn,
@@ -470,26 +472,32 @@ __global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ q
   const int64_t q = blockIdx.x;
   const bool live = q < nq;
   uint8_t* const out = qp + q * (int64_t)(K::kPlanes * KS * 32);
-  bool fractional = false;
+  bool fractional = false, leaves = false;
   if constexpr (K::kFloat) {
-    float s = 0.f;
+    float s = 0.f, x[8];
     if (lane < KS * 2) {
-      float x[8];
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         const int i = lane * 8 + j;
         x[j] = live && i < dim ? queries[q * dim + i] - center[i] : 0.f;
         s = __fmaf_rn(x[j], x[j], s);
       }
+    }
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    leaves = !(s <= kGtHuge);
+    if (lane < KS * 2) {
       gt_b8 hi, lo;
+      if (leaves) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = 0.f;
+      }
       gt_split(x, hi, lo);
       *reinterpret_cast<gt_b8*>(out + lane * 16) = hi;
       *reinterpret_cast<gt_b8*>(out + KS * 32 + lane * 16) = lo;
     }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
     if (lane == 0) {
       qn[q] = __float_as_uint(s);
-      thr[q] = __float_as_uint(live ? -__int_as_float(0x7f800000) : __int_as_float(0x7f800000));
+      thr[q] = live && !leaves ? 0xff800000u : 0x7f800000u;
     }
   } else {
     const float lo = std::is_signed<T>::value ? -128.f : 0.f, hi = std::is_signed<T>::value ? 127.f : 255.f;
@@ -510,7 +518,7 @@ __global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ q
       s = __builtin_amdgcn_sdot4((int)packed, (int)packed, s, false);
       reinterpret_cast<uint32_t*>(out)[w] = packed;
     }
-    fractional = __ballot(wrong) != 0;
+    leaves = fractional = __ballot(wrong) != 0;
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
     if (lane == 0) {
       qn[q] = (uint32_t)s;
@@ -519,11 +527,9 @@ __global__ __launch_bounds__(64) void gt_pack_kernel(const float* __restrict__ q
   }
   if (lane == 0) {
     tkey[q] = kPadKey;
-    cnt[q] = fractional ? kGtLeft : 0u;
-    if (fractional) {
-      call->fractional = 1;
-      gt_leave(left, limit);
-    }
+    cnt[q] = leaves ? kGtLeft : 0u;
+    if (fractional) call->fractional = 1;
+    if (leaves) gt_leave(left, limit);
   }
 }
 
@@ -903,7 +909,7 @@ __global__ __launch_bounds__(256) void gt_pick_kernel(const uint8_t* __restrict_
     const float d = __uint_as_float((uint32_t)(tk >> 32));
     if constexpr (kFloat) {
       // a row is dropped when q.x (the bound) < ((1 - eps)(|q|^2 + |x|^2) - d) / 2;
-      // with no bound for the query (norm or distance not finite) none is
+      // with no bound for the query (distance not finite) none is
       const float n2 = __uint_as_float(qn[q]);
       const double at = 0.5 * ((1.0 - (double)kGtEps) * (double)n2 - (double)d) - 1e-30;
       thr[q] = __float_as_uint(tk != kPadKey && n2 <= kGtHuge && d <= kGtHuge ? __double2float_rd(at)

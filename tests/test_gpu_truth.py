@@ -212,6 +212,28 @@ def test_queries_that_leave_the_scan(lib, what, direct):
     _check(base, q, 10, ids, dists)
 
 
+def test_queries_without_a_norm(lib):
+    """Queries with NaN, infinite or enormous elements leave the scan before it, alone: the others' answers are those
+    of a call without them, and theirs the ones of the direct kernels."""
+    print("[gpu] truth, queries without a norm", flush=True)
+    base, q = _rows("float32", 20000, 96, 5), _rows("float32", 70, 96, 6)
+    want = _counted(lib, base, q, 10)
+    bad = {3: np.nan, 17: np.inf, 18: -np.inf, 60: 1e30, 69: 3e38}
+    for row, v in bad.items():
+        q[row, row] = v
+    got = _counted(lib, base, q, 10)
+    assert (want[2], got[2]) == (0, len(bad))
+    rest = np.array([i for i in range(70) if i not in bad])
+    np.testing.assert_array_equal(got[0][rest], want[0][rest])
+    np.testing.assert_array_equal(got[1][rest], want[1][rest])
+    # a call of few rows is the direct kernels' own: the same rows, repeated past that line, against it
+    few = _counted(lib, base[:2000], q[list(bad)], 10)
+    scanned = _counted(lib, base[:2000], q[list(bad)], 10, 1)
+    assert few[2] == scanned[2] == len(bad)
+    np.testing.assert_array_equal(few[0], scanned[0])
+    np.testing.assert_array_equal(few[1], scanned[1])
+
+
 @pytest.mark.parametrize("dtype", ["uint8", "float32"])
 def test_query_batches(lib, dtype):
     """More queries than one scan takes (32,768): the second batch has its own lists, results and queries that leave."""
