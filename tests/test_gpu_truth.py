@@ -226,7 +226,7 @@ def test_queries_without_a_norm(lib):
     rest = np.array([i for i in range(70) if i not in bad])
     np.testing.assert_array_equal(got[0][rest], want[0][rest])
     np.testing.assert_array_equal(got[1][rest], want[1][rest])
-    # a call of few rows is the direct kernels' own: the same rows, repeated past that line, against it
+    # theirs: a call over few rows is the direct kernels' own; taken by the scan, they leave it and get the same bits
     few = _counted(lib, base[:2000], q[list(bad)], 10)
     scanned = _counted(lib, base[:2000], q[list(bad)], 10, 1)
     assert few[2] == scanned[2] == len(bad)
