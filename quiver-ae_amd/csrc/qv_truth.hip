@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <type_traits>
 
 #include "qv_common.hpp"
@@ -922,6 +923,23 @@ __global__ __launch_bounds__(256) void gt_pick_kernel(const uint8_t* __restrict_
   }
 }
 
+// Memory of a call, given back in its stream's order, also when the call fails.
+struct CallMemory {
+  hipStream_t st;
+  void* p = nullptr;
+  explicit CallMemory(hipStream_t s) : st(s) {}
+  CallMemory(const CallMemory&) = delete;
+  CallMemory& operator=(const CallMemory&) = delete;
+  ~CallMemory() {
+    if (p) (void)hipFreeAsync(p, st);
+  }
+  hipError_t take(size_t bytes) { return hipMallocAsync(&p, bytes, st); }
+  template <class U>
+  U* as() const {
+    return static_cast<U*>(p);
+  }
+};
+
 int grid_of(int64_t work, int block) {
   return (int)std::max<int64_t>(1, std::min<int64_t>((work + block - 1) / block, 1 << 20));
 }
@@ -986,7 +1004,7 @@ void gt_levels(const T* d_base, int64_t n, int dim, const float* d_q, int64_t nq
 template <class T>
 void gt_direct(const T* d_base, int64_t n, int dim, const float* d_q, const int64_t* which, int64_t nq, int k,
                int32_t* d_ids, float* d_dists, bool whole, hipStream_t st) {
-  uint64_t* part = nullptr;
+  CallMemory partial(st);
   int S = 0;
   if (sizeof(T) == 1 && whole && dim <= 4 * kGtWords && k <= kGtMaxK) {
     if constexpr (sizeof(T) == 1) {
@@ -994,23 +1012,22 @@ void gt_direct(const T* d_base, int64_t n, int dim, const float* d_q, const int6
       const int64_t tiles = (n + kGtTile - 1) / kGtTile;
       S = (int)std::max<int64_t>(1, std::min<int64_t>({256, tiles, (2048 + groups - 1) / groups}));
       const int64_t slice = (tiles + S - 1) / S * kGtTile;
-      HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&part), sizeof(uint64_t) * (size_t)(nq * S * k), st));
+      HIP_OK(partial.take(sizeof(uint64_t) * (size_t)(nq * S * k)));
       hipLaunchKernelGGL(gt_int_kernel<T>, dim3((unsigned)groups, (unsigned)S), dim3(256), 0, st, d_base, n, dim, d_q,
-                         which, nq, k, slice, S, part);
+                         which, nq, k, slice, S, partial.as<uint64_t>());
     }
   } else {
     S = (int)std::max<int64_t>(1, std::min<int64_t>(64, 4096 / std::max<int64_t>(1, (nq + kGtQ - 1) / kGtQ)));
     const int64_t slice = (n + S - 1) / S;
-    HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&part), sizeof(uint64_t) * (size_t)(nq * S * k), st));
+    HIP_OK(partial.take(sizeof(uint64_t) * (size_t)(nq * S * k)));
     const size_t lds = (size_t)kGtQ * dim * 4 + (size_t)kGtQ * 4 * kWave * 8;
     hipLaunchKernelGGL(gt_kernel<T>, dim3((unsigned)((nq + kGtQ - 1) / kGtQ), (unsigned)S), dim3(256), lds, st, d_base,
-                       n, dim, d_q, which, nq, k, slice, S, part);
+                       n, dim, d_q, which, nq, k, slice, S, partial.as<uint64_t>());
   }
   HIP_OK(hipGetLastError());
-  hipLaunchKernelGGL(gt_final_kernel, dim3((unsigned)std::min<int64_t>(nq, 65536)), dim3(64), 0, st, part, which, nq, S,
-                     k, d_ids, d_dists);
+  hipLaunchKernelGGL(gt_final_kernel, dim3((unsigned)std::min<int64_t>(nq, 65536)), dim3(64), 0, st,
+                     partial.as<uint64_t>(), which, nq, S, k, d_ids, d_dists);
   HIP_OK(hipGetLastError());
-  HIP_OK(hipFreeAsync(part, st));
 }
 
 // The whole call by the scan, then the direct kernels for the queries that
@@ -1029,14 +1046,14 @@ bool gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t
   const int64_t padded = (batch + 128 * QT - 1) / (128 * QT) * (128 * QT);
   const size_t lists = (size_t)batch * cap * 8 + (size_t)padded * (8 + 12 + GtKind<T>::kPlanes * KS * 32);
   const size_t state = sizeof(GtCall) + (size_t)batches * sizeof(GtLeft);
-  uint8_t* work = nullptr;
-  const hipError_t got =
-      hipMallocAsync(reinterpret_cast<void**>(&work), lists + state + (size_t)nq * 8 + kGtCenter * 4, st);
+  CallMemory memory(st);
+  const hipError_t got = memory.take(lists + state + (size_t)nq * 8 + kGtCenter * 4);
   if (got == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     return false;
   }
   HIP_OK(got);
+  uint8_t* const work = memory.as<uint8_t>();
   GtCall* const call = reinterpret_cast<GtCall*>(work + lists);
   GtLeft* const left = reinterpret_cast<GtLeft*>(call + 1);
   int64_t* const listed = reinterpret_cast<int64_t*>(left + batches);
@@ -1055,7 +1072,6 @@ bool gt_matrix_ks(const T* d_base, int64_t n, int dim, const float* d_q, int64_t
     gt_direct<T>(d_base, n, dim, d_q, listed, (int64_t)host.direct, k, d_ids, d_dists, !host.fractional, st);
     HIP_OK(hipStreamSynchronize(st));
   }
-  HIP_OK(hipFreeAsync(work, st));
   return true;
 }
 
@@ -1118,15 +1134,14 @@ void ground_truth_t(const T* d_base, int64_t n, int dim, const float* d_q, int64
   int32_t bad = 1;
   if constexpr (sizeof(T) == 1) {
     if (dim <= 4 * kGtWords && k <= kGtMaxK) {
-      int32_t* d_bad = nullptr;
-      HIP_OK(hipMallocAsync(reinterpret_cast<void**>(&d_bad), sizeof(int32_t), st));
-      HIP_OK(hipMemsetAsync(d_bad, 0, sizeof(int32_t), st));
+      CallMemory flag(st);
+      HIP_OK(flag.take(sizeof(int32_t)));
+      HIP_OK(hipMemsetAsync(flag.p, 0, sizeof(int32_t), st));
       hipLaunchKernelGGL(gt_query_check<T>, dim3((unsigned)grid_of(nq * dim, 256)), dim3(256), 0, st, d_q, nq * dim,
-                         d_bad);
+                         flag.as<int32_t>());
       HIP_OK(hipGetLastError());
-      HIP_OK(hipMemcpyAsync(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost, st));
+      HIP_OK(hipMemcpyAsync(&bad, flag.p, sizeof(bad), hipMemcpyDeviceToHost, st));
       HIP_OK(hipStreamSynchronize(st));
-      HIP_OK(hipFreeAsync(d_bad, st));
     }
   }
   gt_direct<T>(d_base, n, dim, d_q, nullptr, nq, k, d_ids, d_dists, !bad, st);
@@ -1147,13 +1162,14 @@ int qv_ground_truth_counted(const void* d_base, int32_t data_type, int64_t n, in
     HIP_OK(hipSetDevice(device));
     hipStream_t st;
     HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    std::unique_ptr<std::remove_pointer<hipStream_t>::type, void (*)(hipStream_t)> owned(
+        st, [](hipStream_t s) { (void)hipStreamDestroy(s); });
     auto go = [&](auto* base) {
       ground_truth_t(base, n, dim, d_queries, nq, k, d_ids, d_dists, device, scan_small != 0, direct, st);
     };
     if (data_type == QV_UINT8) go(static_cast<const uint8_t*>(d_base));
     else if (data_type == QV_INT8) go(static_cast<const int8_t*>(d_base));
     else go(static_cast<const float*>(d_base));
-    HIP_OK(hipStreamDestroy(st));
   });
 }
 

@@ -6,7 +6,8 @@
 //                             every i the call reaches, fails and frees
 //                             nothing twice
 //   alloc_failure_test truth  ground truth whose first allocation (the matrix
-//                             scan's lists) is refused still runs
+//                             scan's lists) is refused still runs, and whichever
+//                             is refused leaves no memory and no stream behind
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
@@ -24,6 +25,7 @@ long allocs = 0;            // allocations asked for
 long refuse = 0;            // the one to refuse (from 1; 0: none)
 long double_frees = 0;
 long launches = 0;
+long streams = 0;           // created and not destroyed
 
 hipError_t take(void** p, size_t bytes) {
   *p = nullptr;
@@ -59,8 +61,11 @@ int hipGetStreamDeviceId(hipStream_t) { return 0; }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
-hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = reinterpret_cast<hipStream_t>(8), hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = reinterpret_cast<hipStream_t>(8);
+  return streams++, hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return streams--, hipSuccess; }
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(8), hipSuccess; }
@@ -122,7 +127,7 @@ static int build_refused() {
 }
 
 static int truth_refused() {
-  const int64_t n = 5000, nq = 20;
+  const int64_t n = 5000, nq = 300;
   const int32_t dim = 32, k = 50;
   std::vector<float> base((size_t)n * dim, 1.f), q((size_t)nq * dim, 2.f), dists((size_t)nq * k);
   std::vector<int32_t> ids((size_t)nq * k);
@@ -134,6 +139,19 @@ static int truth_refused() {
         std::printf("type %d, allocation %ld refused: status %d (%s), %ld launches, %zu allocations left\n", type, refuse,
                     rc, qv_last_error(), launches, live.size());
         return 1;
+      }
+    }
+    // few rows: the direct kernels' own check and partial results
+    for (int32_t kk : {10, 50}) {
+      for (refuse = 1;; refuse++) {
+        allocs = 0;
+        const int rc = qv_ground_truth(base.data(), type, 100, dim, q.data(), nq, kk, ids.data(), dists.data(), 0);
+        if (!live.empty() || streams != 0 || double_frees != 0 || (rc != QV_OK && rc != QV_ENOMEM)) {
+          std::printf("type %d, k %d, allocation %ld refused: status %d (%s), %zu allocations and %ld streams left\n", type,
+                      kk, refuse, rc, qv_last_error(), live.size(), streams);
+          return 1;
+        }
+        if (allocs < refuse) break;
       }
     }
   }
